@@ -873,6 +873,149 @@ def test_gemm_epilogue(torch):
                 (A @ B + C0) + bn)
 
 
+def _raw_split(torch, ta, tb, A, B, M, N, K, alpha=1.0, beta=0.0, C0=None, bias=None, bmode=0,
+               res=None, act=0, shift=0):
+    """tjh_gemm_split on op(A) and op(B) as stored, `shift` floats into
+    their buffers."""
+    from torchjs_amd import _lib as L
+    a, b = (torch.tensor(np.concatenate([np.zeros(shift, np.float32), x.ravel()])) for x in (A, B))
+    c = torch.tensor(C0 if C0 is not None else np.zeros((M, N), np.float32))
+    bb = torch.tensor(bias) if bias is not None else None
+    r = torch.tensor(res) if res is not None else None
+    L.check(L.lib().tjh_gemm_split(ta, tb, M, N, K, alpha, a.data_ptr() + 4 * shift, A.shape[1],
+                                   b.data_ptr() + 4 * shift, B.shape[1], beta, c.data_ptr(), N,
+                                   bb.data_ptr() if bb else None, bmode,
+                                   r.data_ptr() if r else None, N, act))
+    return c.numpy()
+
+
+SPLIT_TILES = ["256x256", "256x192", "256x128", "128x128", "128x64", "64x64"]
+
+
+@pytest.mark.parametrize("tile", SPLIT_TILES)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,shift", [(300, 260, 200, 0), (256, 384, 4096, 0), (5, 3, 35, 1),
+                                         (257, 193, 541, 3), (130, 129, 31, 0)])
+def test_gemm_split_every_tile(torch, monkeypatch, tile, ta, tb, M, N, K, shift):
+    """Whole tiles, tiles over both edges, K tails, slices of K, operands off
+    16-byte alignment, and the products left to the float cores (K < 32,
+    both operands transposed)."""
+    monkeypatch.setenv("TJH_SPLIT_TILE", tile)
+    r = np.random.default_rng(M + N + K + ta * 2 + tb)
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    bias, C0 = f32(r.standard_normal(N)), f32(r.standard_normal((M, N)))
+    want = 0.5 * (A.astype(np.float64) @ B.astype(np.float64)) + 0.25 * C0 + bias
+    got = _raw_split(torch, ta, tb, np.ascontiguousarray(A.T) if ta else A,
+                     np.ascontiguousarray(B.T) if tb else B, M, N, K, 0.5, 0.25, C0, bias, 1,
+                     shift=shift)
+    check_floor(got, want, np.float32(0.5) * (A @ B) + np.float32(0.25) * C0 + bias)
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 90, 50), (512, 384, 768), (64, 96, 6000)])
+def test_gemm_split_epilogues(torch, M, N, K):
+    """GELU and residual epilogues, column and row bias, in one slice and
+    with K in several."""
+    r = np.random.default_rng(M)
+    A, B = f32(r.standard_normal((M, K)) / np.sqrt(K)), f32(r.standard_normal((K, N)))
+    bias, bm, res = (f32(r.standard_normal(n)) for n in (N, M, (M, N)))
+    z = A.astype(np.float64) @ B.astype(np.float64)
+    check(_raw_split(torch, 0, 0, A, B, M, N, K, bias=bias, bmode=1, act=1),
+          ops.unary("gelu", z + bias), **RED)
+    check(_raw_split(torch, 0, 0, A, B, M, N, K, act=1), ops.unary("gelu", z), **RED)
+    check(_raw_split(torch, 0, 0, A, B, M, N, K, bias=bias, bmode=1, res=res, act=3),
+          z + bias + res, **RED)
+    check(_raw_split(torch, 0, 0, A, B, M, N, K, bias=bm, bmode=2), z + bm[:, None], **RED)
+
+
+@pytest.mark.parametrize("tile", SPLIT_TILES)
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0)])
+def test_gemm_split_not_finite_every_tile(torch, monkeypatch, tile, ta, tb):
+    """Infinities, NaNs and floats above the largest bfloat16 give the sums
+    of float arithmetic, where they stand and nowhere else."""
+    monkeypatch.setenv("TJH_SPLIT_TILE", tile)
+    r = np.random.default_rng(len(tile) + ta)
+    M, N, K = 300, 270, 70
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    A[3, 5], A[130, 69], B[0, 200] = np.inf, -np.inf, np.nan
+    A[257, :], A[257, 2] = 0, 3.4e38  # rounds to infinity in bfloat16
+    A[40, 7], B[7, 11] = np.inf, 0  # inf * 0
+    got = _raw_split(torch, ta, tb, np.ascontiguousarray(A.T) if ta else A,
+                     np.ascontiguousarray(B.T) if tb else B, M, N, K)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = A.astype(np.float64) @ B.astype(np.float64)
+        want32 = want.astype(np.float32)
+        # a one-term row: its product alone, infinite only where a float is
+        want32[257] = A[257, 2] * B[2]
+    want32[:, 200] = np.nan
+    assert np.array_equal(np.isnan(got), np.isnan(want32))
+    assert np.array_equal(np.isinf(got), np.isinf(want32))
+    inf = np.isinf(want32)
+    assert np.array_equal(got[inf], want32[inf])
+    ok = np.isfinite(want32) & np.isfinite(want)
+    ok[257] = False
+    check(got[ok], want[ok], **RED)
+    fin = np.isfinite(want32[257])
+    assert np.array_equal(got[257][fin], want32[257][fin])
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 512, 768), (200, 300, 1000), (64, 64, 8192)])
+def test_gemm_split_error_of_float_products(torch, M, N, K):
+    """Against 64 bits the three-part products are no further off than a
+    chain of float multiply-adds, and their errors do not drift: the mean
+    error of a product is within 5 standard errors of zero."""
+    r = np.random.default_rng(M + N + K)
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    chain = np.zeros((M, N), np.float32)
+    for k in range(K):  # the sum in doubles, rounded: a fused multiply-add
+        chain = (chain + A[:, k, None].astype(np.float64) * B[k].astype(np.float64)).astype(np.float32)
+    err = _raw_split(torch, 0, 0, A, B, M, N, K) - want
+    assert np.linalg.norm(err) <= np.linalg.norm(chain - want)
+    assert abs(err.mean()) <= 5 * err.std() / np.sqrt(err.size)
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e30])
+def test_gemm_split_error_of_scaled_operands(torch, scale):
+    """The three parts hold every bit of a float down to 2^-109: 256 terms
+    err by no more than 256 roundings' root sum of squares, 16 x 2^-24 / 2."""
+    r = np.random.default_rng(5)
+    M, N, K = 128, 128, 256
+    A = f32(r.standard_normal((M, K)) * scale)
+    B = f32(r.standard_normal((K, N)))
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    got = _raw_split(torch, 0, 0, A, B, M, N, K)
+    assert np.linalg.norm(got - want) <= 4.8e-7 * np.linalg.norm(want)
+
+
+def test_products_without_gradient_take_the_split_kernels(torch):
+    """Linear, the residual and MLP forms and matmul: split products exactly
+    where nothing is recorded, equal to the recorded ones within rounding."""
+    from torchjs_amd import _lib as L, workloads as W
+    real, calls = L.lib().tjh_gemm_split, []
+    blk = W.Block(64, 2)
+    x = torch.tensor(f32(np.random.default_rng(1).standard_normal((2, 40, 64))))
+
+    class Spy:
+        def __getattr__(self, n):
+            return getattr(real_lib, n)
+
+        def tjh_gemm_split(self, *a):
+            calls.append(a[2:5])
+            return real(*a)
+    real_lib = L._lib
+    try:
+        L._lib = Spy()
+        y = blk(x).numpy()
+        assert not calls
+        with torch.no_grad():
+            z = blk(x).numpy()
+            (x.reshape(80, 64) @ x.reshape(80, 64).t()).numpy()
+    finally:
+        L._lib = real_lib
+    assert len(calls) == 5
+    check(z, y, **RED)
+
+
 def test_matmul_autograd_batched_broadcast(torch):
     r = np.random.default_rng(14)
     a = f32(r.standard_normal((2, 3, 4, 5)))

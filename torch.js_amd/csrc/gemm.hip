@@ -38,8 +38,7 @@
 // order so the sharing happens inside one L2.
 
 #include "colsum.h"
-#include "common.h"
-#include "ops_math.h"
+#include "gemm_args.h"
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -47,64 +46,6 @@
 
 namespace tjh {
 namespace {
-
-constexpr int BK = 16;
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-// Staging registers are native 4-wide vectors: a struct float4 copied out
-// of a reinterpret_cast load is not always split into registers by the
-// compiler and then lives in scratch memory.
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-// The same vector at 4-byte alignment: operand rows start wherever the row
-// stride puts them.
-typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
-
-struct GemmArgs {
-  const float* A;
-  const float* B;
-  float* C;
-  const float* bias;
-  int64_t M, N, K;
-  int64_t lda, ldb, ldc;
-  int64_t sA, sB, sC;
-  float alpha, beta;
-  int bias_mode;
-  int vecA, vecB;  // 128-bit loads allowed for the operand
-  int tiles_m, tiles_n;
-  int64_t kchunk;  // K range per split (multiple of BK); splits = gridDim.y
-  float* ws;       // split-K partials [batch][split][M][N] (nullptr: none)
-  float* rsw;      // split-K partials of the row sums (bias_mode 3/4) [split][M]
-  // epilogue activation on the final C values (after alpha, beta, bias):
-  // 1: aux <- v, C <- GELU(v);  2: C <- v * GELU'(aux);  3: C <- aux + v
-  float* aux;
-  int64_t ldaux;
-  int act;
-  // A formed on load from logits (k_gemm<..., XF>): A's element at logits
-  // row r, class c is (exp(logits[r][c] - lse_r) - (c == t_r)) * s_r, the
-  // cross-entropy gradient, with xrow[r] = {lse_r, s_r, t_r (int bits), 0};
-  // xm0 / xk0 locate this (sub-)product in the logits (rows = m without
-  // TA, k with TA)
-  const floatx4* xrow;
-  int64_t xm0, xk0;
-};
-
-// A compile-time int carried by a value (dispatch into generic lambdas).
-template <int V>
-struct IConst {
-  static constexpr int value = V;
-};
-
-// The activation epilogue, shared by the GEMM and the split-K sum.
-__device__ __forceinline__ float epilogue_act(const GemmArgs& g, int64_t row, int64_t col,
-                                              float v) {
-  if (g.act == 1) {
-    g.aux[row * g.ldaux + col] = v;
-    return gelu_f(v);
-  }
-  if (g.act == 2) return v * gelu_grad(g.aux[row * g.ldaux + col]);
-  if (g.act == 3) return g.aux[row * g.ldaux + col] + v;
-  return v;
-}
 
 // Loads a logical OUTER x BK tile (outer = m for A, n for B) for this lane:
 // V float4 per lane.  !TRANS: storage [outer][k] (k contiguous, 4 float4
@@ -893,16 +834,7 @@ int run_block(int ti, GemmArgs g, int ta, int tb, int64_t splits, int64_t batch,
   launch_tile(ti, g, grid, ta, tb, edge);
   int rc = check_launch("gemm");
   if (rc != TJH_OK || splits == 1) return rc;
-  const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && g.sC % 4 == 0 && aligned16(g.C);
-  int64_t blocks = cdiv(g.M * g.N / (vec ? 4 : 1), 256);
-  if (blocks > 16LL * cus) blocks = 16LL * cus;
-  if (vec)
-    tjh_launch(k_splitk_reduce<true>, dim3((unsigned)blocks, (unsigned)batch), dim3(256),
-                       0, stream(), g, (int)splits);
-  else
-    tjh_launch(k_splitk_reduce<false>, dim3((unsigned)blocks, (unsigned)batch), dim3(256),
-                       0, stream(), g, (int)splits);
-  return check_launch("gemm_splitk_reduce");
+  return gemm_splitk_sum(g, splits, batch, cus);
 }
 
 // Sub-problem of g: rows [m0, m0+M), cols [n0, n0+N), k [k0, k0+K).
@@ -922,6 +854,20 @@ GemmArgs sub(const GemmArgs& g, int ta, int tb, int64_t m0, int64_t M, int64_t n
 }
 
 }  // namespace
+
+int gemm_splitk_sum(const GemmArgs& g, int64_t splits, int64_t batch, int cus) {
+  const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && g.sC % 4 == 0 && aligned16(g.C);
+  int64_t blocks = cdiv(g.M * g.N / (vec ? 4 : 1), 256);
+  if (blocks > 16LL * cus) blocks = 16LL * cus;
+  if (vec)
+    tjh_launch(k_splitk_reduce<true>, dim3((unsigned)blocks, (unsigned)batch), dim3(256),
+                       0, stream(), g, (int)splits);
+  else
+    tjh_launch(k_splitk_reduce<false>, dim3((unsigned)blocks, (unsigned)batch), dim3(256),
+                       0, stream(), g, (int)splits);
+  return check_launch("gemm_splitk_reduce");
+}
+
 }  // namespace tjh
 
 using namespace tjh;

@@ -1,0 +1,543 @@
+// fp32 GEMM on the CDNA4 bf16 matrix cores: products of floats split into
+// three bf16 parts.  Serves the products that no gradient is taken through
+// (tjh_gemm_split); gemm.hip's float matrix cores serve the recorded ones,
+// whose roundings a training run depends on: AdamW's g / (|g| + eps)
+// amplifies any change of them to 2e-5 in the second step's gradients of
+// GPT-2, in which the float path itself is 1.6e-5 from 64 bits.
+//
+// Stands for matmul.wgsl:17-50 behind Tensor.matmul / mm and nn.Linear
+// (Tensor.ts:2132-2331, src/nn/linear.ts:43-66) under no_grad.
+//
+// C = alpha * op(A) op(B) + beta * C (+ bias), row-major.
+//
+// Products.  v_mfma_f32_32x32x2_f32 does 64 FLOP per cycle and SIMD, the
+// bf16 32x32x16 form 1024.  Each float is split into three bf16 parts that
+// sum to it exactly (split2 below) and six of the nine part products are
+// added up in float: 2.67 times the float rate, with an error against 64
+// bits under the float form's (a 768-term product of normal values: 4.2e-7
+// against 5.0e-7 rel.; 8192 terms: 1.45e-6 against 1.7e-6), because a
+// 16-term step meets fewer roundings.  8192 x 3072 x 768 takes 317-350 us on
+// the float cores and 193-240 us here, 8192 x 768 x 50257 4.7 and 3.4 ms,
+// 777 x 2304 x 768 50 and 30 us.  What bounds the large ones is power: with
+// random operands the clock falls to 1.9 GHz (an all-zero product runs at
+// 2.36 GHz and 309 TFLOP/s, a random one of 8192^3 at 214-238), so data
+// moved per product counts as much as issue slots.
+//
+// Tiling (a workgroup of WR x WC waves): block tile BM x BN, K step 16; each
+// wave owns a (BM / WR) x (BN / WC) sub-tile of 32x32 MFMA blocks.  Operand
+// tiles are loaded as floats into registers one step ahead (two steps on
+// wave tiles of 64 x 64 or less, which have the registers: 250 -> 214 us for
+// 8192 x 3072 x 768 on 128 x 128), split there once per workgroup, and
+// stored as three planes of bf16 in one of two LDS buffers.  The larger wave
+// tiles read and split less per product but leave CUs idle on small outputs:
+//   256 x 256, 8 waves of 128 x 64, one workgroup per CU
+//   256 x 192, 8 waves of 64 x 96, one per CU
+//   256 x 128, 4 waves of 128 x 64, two per CU
+//   128 x 128 / 128 x 64 / 64 x 64, 4 waves, three or more per CU
+// Small outputs with long K are split over K; partials are summed by a
+// second pass in a fixed order (deterministic).
+// MFMA operand layout (32x32x16 bf16): lane l feeds A[m = l%32][k = 8*(l/32)
+//   + 0..7] and B[the same k][n = l%32]; accumulator register r of lane l
+//   holds C[8*(r/4) + 4*(l/32) + r%4][l%32].
+// Operand loads are 128-bit along k, or a wave's 256 consecutive bytes and
+// more along the outer index, at any 4-byte alignment (HSA runs the GPU in
+// unaligned-access mode; the compiler itself emits such loads for packed
+// data), so odd row strides need nothing of their own.  Tiles over the edge
+// of the product repeat its last row or column and do not store it; a last K
+// step of fewer than 16 is loaded float by float.
+// Workgroup order: tiles are grouped 8 M-tiles at a time so neighbouring
+// tiles share B columns, and each XCD receives a contiguous run of that
+// order so the sharing happens inside one L2.
+
+#pragma once
+
+#include "gemm_args.h"
+
+namespace tjh {
+
+// ------------------------------------------------------- the operand split
+
+// A float as three bfloat16 parts: x = h + m + l, each part the nearest
+// bfloat16 of what is left.  Three times eight significant bits hold the 24
+// of a float: the sum is exact while the parts stay above the smallest
+// bfloat16 (2^-133), so for |x| >= 2^-109; below, an absolute error of at
+// most 2^-134 remains.  |m| <= 2^-9 |x| and |l| <= 2^-18 |x|, so of the
+// nine products of two split numbers the three not formed (m l, l m, l l)
+// are under 2^-26 of the product, a quarter of one float rounding.
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
+}
+__device__ __forceinline__ float bf16_lo(unsigned u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float bf16_hi(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
+// the parts of sign * a and sign * b, packed (the differences are exact)
+__device__ __forceinline__ void split2(float a, float b, float sign, unsigned& h, unsigned& m,
+                                       unsigned& l) {
+  h = pack_bf16(a, b) ^ (sign < 0.f ? 0x80008000u : 0u);
+  const float ra = __builtin_fmaf(a, sign, -bf16_lo(h)), rb = __builtin_fmaf(b, sign, -bf16_hi(h));
+  m = pack_bf16(ra, rb);
+  l = pack_bf16(ra - bf16_lo(m), rb - bf16_hi(m));
+}
+
+// LDS layout of one part of an operand tile: per 32 outer indices (m or n)
+// a kBlk-byte block of 16-byte chunks (8 k values of one outer index), in
+// the order the MFMA reads them: lane l takes outer index l % 32, k = 8
+// (l / 32) .. + 7, so a fragment is one contiguous 1 KB read.  The chunks of
+// the second k half are rotated by four so that a wave storing both halves
+// of neighbouring rows does not meet itself in the LDS banks.
+constexpr int kBlk = BK * 32 * 2;
+__device__ __forceinline__ int chunk_at(int o, int kq) {
+  return (o >> 5) * kBlk + kq * 512 + ((o & 31) ^ (kq << 2)) * 16;
+}
+
+// An operand tile of OUTER x BK floats in the registers of T lanes, as items
+// of 8 k values x W outer indices.  KC: the operand is stored [outer][k]
+// (k contiguous); otherwise [k][outer], and a wave's items share their k
+// rows, so a row's address is uniform.  The last pass over the lanes may
+// cover part of the workgroup's waves.
+// EDGE: outer indices past the end repeat the last one (their products are
+// never stored), one at a time.
+template <bool KC, int OUTER, int T, bool EDGE>
+struct Tile {
+  static constexpr int W = !KC && !EDGE && OUTER * BK / 8 / T >= 2 ? 2 : 1;
+  static constexpr int NI = OUTER * BK / 8 / W;  // items of the tile
+  static constexpr int I = (NI + T - 1) / T;     // items per lane
+  static_assert(BK == 16 && NI % 64 == 0 && (KC || OUTER / W % 64 == 0), "whole waves");
+  float r[I][W][8];
+
+  __device__ __forceinline__ static bool has(int i) {
+    return NI % T == 0 || (int)threadIdx.x + T * i < NI;
+  }
+  __device__ __forceinline__ static void at(int i, int& o, int& kq) {
+    const int f = threadIdx.x + T * i;
+    if (KC) {
+      o = f >> 1;
+      kq = f & 1;
+    } else {
+      constexpr int Q = OUTER / W;
+      kq = __builtin_amdgcn_readfirstlane(f / Q);
+      o = (f % Q) * W;
+    }
+  }
+  // Loads the whole K tile at outer index o0, k index k0 of P (row stride
+  // ld, `rows` outer indices).
+  __device__ __forceinline__ void load(const float* __restrict__ P, int64_t ld, int64_t rows,
+                                       int64_t o0, int64_t k0) {
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      if (!has(i)) continue;
+      int o, kq;
+      at(i, o, kq);
+      if (EDGE && o0 + o >= rows) o = (int)(rows - 1 - o0);
+      if (KC) {
+        const float* __restrict__ p = P + (o0 + o) * ld + k0 + kq * 8;
+        const floatx4 a = *reinterpret_cast<const floatx4u*>(p);
+        const floatx4 b = *reinterpret_cast<const floatx4u*>(p + 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          r[i][0][k] = a[k];
+          r[i][0][4 + k] = b[k];
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const float* __restrict__ p = P + (k0 + kq * 8 + k) * ld + o0;
+          if (W == 2) {
+            const floatx2 v = *reinterpret_cast<const floatx2u*>(p + (unsigned)o);
+            r[i][0][k] = v.x;
+            r[i][W - 1][k] = v.y;
+          } else {
+            r[i][0][k] = p[(unsigned)o];
+          }
+        }
+      }
+    }
+  }
+  // The same float by float, with 0 for k past kend.
+  __device__ __forceinline__ void load_tail(const float* __restrict__ P, int64_t ld, int64_t rows,
+                                            int64_t kend, int64_t o0, int64_t k0) {
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      if (!has(i)) continue;
+      int o, kq;
+      at(i, o, kq);
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const int64_t go = o0 + o + w < rows ? o0 + o + w : rows - 1;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int64_t gk = k0 + kq * 8 + k;
+          r[i][w][k] = gk < kend ? (KC ? P[go * ld + gk] : P[gk * ld + go]) : 0.f;
+        }
+      }
+    }
+  }
+  // Splits the tile and stores its parts in LDS, `part` bytes apart, outer
+  // index o negated where o + flip is odd (kFlip below).
+  __device__ __forceinline__ void store(char* __restrict__ S, int part, int flip) const {
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      if (!has(i)) continue;
+      int o, kq;
+      at(i, o, kq);
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const float sign = (o + w + flip) & 1 ? -1.f : 1.f;
+        uintx4 h, m, l;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          unsigned a, b, c;
+          split2(r[i][w][2 * q], r[i][w][2 * q + 1], sign, a, b, c);
+          h[q] = a;
+          m[q] = b;
+          l[q] = c;
+        }
+        char* d = S + chunk_at(o + w, kq);
+        *reinterpret_cast<uintx4*>(d) = h;
+        *reinterpret_cast<uintx4*>(d + part) = m;
+        *reinterpret_cast<uintx4*>(d + 2 * part) = l;
+      }
+    }
+  }
+};
+
+// Workgroups are dispatched to the 8 XCDs round-robin (workgroup w runs on
+// XCD w % 8), and each XCD has its own L2.  Renumbering so that XCD x
+// receives the contiguous run [x*n/8, (x+1)*n/8) of the grouped tile order
+// keeps the tiles that share A rows and B columns on one L2.  A bijection on
+// [0, n): ids past the last multiple of 8 keep their number.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_tile(int bid, int n) {
+  const int full = n - n % kXcds;
+  if (bid >= full) return bid;
+  return (bid % kXcds) * (full / kXcds) + bid / kXcds;
+}
+
+// Wave tiles that keep 96 accumulator registers or more run two waves per
+// SIMD (256 registers each), smaller ones three or more.
+constexpr int gemm_waves_per_simd(int wm, int wn) { return wm * wn >= 64 * 96 ? 2 : wm * wn >= 64 * 64 ? 3 : 4; }
+
+// The bf16 matrix cores round their sums down (toward minus infinity), not
+// to the nearest, so a long sum drifts and so does the mean of a product (43
+// standard errors for 8192 x 3072 x 768).  Two changes of sign undo it:
+//   every second row of A and column of B is negated, so that the sums of
+//   neighbouring elements round in opposite directions;
+//   every kFlip K tiles the running sums and the signs of A are negated, so
+//   that a sum meets both directions.
+constexpr int kFlip = 32;
+
+template <int BM, int BN, int WR, int WC, bool TA, bool TB, bool EDGE>
+__global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)) void k_gemm_split(
+    GemmArgs g) {
+  constexpr int T = WR * WC * 64;
+  constexpr int WM = BM / WR, WN = BN / WC;  // wave tile
+  constexpr int FM = WM / 32, FN = WN / 32;  // MFMA blocks per wave
+  constexpr int PA = BM * BK * 2, PB = BN * BK * 2, BUF = 3 * (PA + PB);
+  static_assert(FM >= 1 && FN >= 1 && FM * 32 == WM && FN * 32 == WN, "tile");
+  __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
+
+  // Wave priority: the prologue and the epilogue run at raised priority.
+  // Where two workgroups share a CU, at equal priority the one in its
+  // epilogue (address arithmetic and stores) barely advances while the
+  // other issues MFMAs, and its successor cannot start.
+  __builtin_amdgcn_s_setprio(3);
+  // ---- tile coordinates (grouped ordering for L2 reuse)
+  const int tiles_m = g.tiles_m, tiles_n = g.tiles_n;
+  int bid = xcd_tile(blockIdx.x, gridDim.x);
+  constexpr int GROUP = 8;
+  int group_size = GROUP * tiles_n;
+  int group = bid / group_size;
+  int first_m = group * GROUP;
+  int gm = tiles_m - first_m < GROUP ? tiles_m - first_m : GROUP;
+  int in_group = bid % group_size;
+  int tm = first_m + in_group % gm;
+  int tn = in_group / gm;
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+
+  const float* __restrict__ A = g.A;
+  const float* __restrict__ B = g.B;
+  float* __restrict__ C = g.C;
+  // split-K: this workgroup covers K range [kbeg, kend)
+  const int64_t kbeg = (int64_t)blockIdx.y * g.kchunk;
+  const int64_t kend = kbeg + g.kchunk < g.K ? kbeg + g.kchunk : g.K;
+
+  const int lane = threadIdx.x & 63;
+  const int wid = threadIdx.x >> 6;
+  const int wm = wid / WC, wn = wid % WC;
+  const int l32 = lane & 31, h = lane >> 5;
+
+  floatx16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  // A: logical [M][K]; stored [M][K] (!TA) or [K][M] (TA)
+  // B: logical [K][N]; as an "outer = n" tile it is stored [N][K] when TB
+  //    (k contiguous, like !TA) and [K][N] when !TB (n contiguous, like TA).
+  // `ktiles` whole K tiles; the rest (fewer than BK k values, or all of them
+  // where the operands are not 4-byte aligned) is loaded float by float
+  const int64_t ktiles = kend > kbeg && (!EDGE || (g.vecA && g.vecB)) ? (kend - kbeg) / BK : 0;
+  using TileA = Tile<!TA, BM, T, EDGE>;
+  using TileB = Tile<TB, BN, T, EDGE>;
+  TileA ta, ta2;
+  TileB tb, tb2;
+  auto fetch = [&](int64_t t, TileA& xa, TileB& xb) {
+    const int64_t k0 = kbeg + t * BK;
+    xa.load(A, g.lda, g.M, m0, k0);
+    xb.load(B, g.ldb, g.N, n0, k0);
+  };
+  auto stage = [&](int64_t t, TileA& xa, TileB& xb) {
+    char* S = lds + (t & 1) * BUF;
+    xa.store(S, PA, (int)(t / kFlip) & 1);
+    xb.store(S + 3 * PA, PB, 0);
+  };
+  // The six products of a K tile, the smallest terms first: the rounding of
+  // the running sum is the only float rounding they meet.
+  auto compute = [&](int64_t t) {
+    if (t % kFlip == 0 && t > 0) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = -acc[i][j];
+    }
+    const char* S = lds + (t & 1) * BUF;
+    const int at = (h << 9) + ((l32 ^ (h << 2)) << 4);
+    const char* as = S + wm * FM * kBlk + at;
+    const char* bs = S + 3 * PA + wn * FN * kBlk + at;
+    constexpr int PI[6] = {2, 1, 0, 1, 0, 0}, PJ[6] = {0, 1, 2, 0, 1, 0};
+    bf16x8 bf[FN][3];
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        bf[j][p] = *reinterpret_cast<const bf16x8*>(bs + p * PB + j * kBlk);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      bf16x8 af[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        af[p] = *reinterpret_cast<const bf16x8*>(as + p * PA + i * kBlk);
+#pragma unroll
+      for (int u = 0; u < 6; ++u)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[PI[u]], bf[j][PJ[u]], acc[i][j],
+                                                              0, 0, 0);
+    }
+  };
+
+  // PF2: two K tiles in flight in registers (tile t + 2 is fetched while
+  // tile t's MFMAs run), for the wave tiles whose registers allow it
+  constexpr bool PF2 = gemm_waves_per_simd(WM, WN) > 2;
+  if (ktiles > 0) {
+    fetch(0, ta, tb);
+    if (PF2 && ktiles > 1) fetch(1, ta2, tb2);
+    stage(0, ta, tb);
+  }
+  __syncthreads();
+  __builtin_amdgcn_s_setprio(0);
+  // The scheduling barriers keep the loads ahead of the MFMAs (the
+  // scheduler sinks them to shorten their registers' lifetimes).
+  if constexpr (PF2) {
+    const int64_t last = ktiles - 1;
+    int64_t t = 0;
+    for (; t + 1 < ktiles; t += 2) {  // two steps per pass keep the sets static
+      fetch(t + 2 < last ? t + 2 : last, ta, tb);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(t);
+      stage(t + 1, ta2, tb2);
+      __syncthreads();
+      fetch(t + 3 < last ? t + 3 : last, ta2, tb2);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(t + 1);
+      if (t + 2 < ktiles) stage(t + 2, ta, tb);
+      __syncthreads();
+    }
+    if (t < ktiles) {
+      compute(t);
+      __syncthreads();
+    }
+  } else {
+    for (int64_t t = 0; t < ktiles; ++t) {
+      const bool more = t + 1 < ktiles;
+      if (more) fetch(t + 1, ta, tb);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(t);
+      if (more) stage(t + 1, ta, tb);
+      __syncthreads();
+    }
+  }
+
+  if constexpr (EDGE) {
+    for (int64_t t = ktiles; kbeg + t * BK < kend; ++t) {
+      const int64_t k0 = kbeg + t * BK;
+      ta.load_tail(A, g.lda, g.M, kend, m0, k0);
+      tb.load_tail(B, g.ldb, g.N, kend, n0, k0);
+      stage(t, ta, tb);
+      __syncthreads();
+      compute(t);
+      __syncthreads();
+    }
+  }
+
+  __builtin_amdgcn_s_setprio(3);
+
+  // ---- epilogue
+  // Element (i, j, r) of this wave sits at row r0 + ro(i, r), column
+  // c0 + 32 j, with ro = 32 i + 8 (r / 4) + r % 4.  Addresses are one base
+  // per lane plus a uniform row offset (ro x ld, scalar arithmetic), and
+  // the beta / bias / activation choice is made once, not per element:
+  // the epilogue runs beside the other workgroup's MFMAs, where every
+  // vector instruction it issues is slow.
+  const int64_t r0 = m0 + wm * WM + 4 * h, c0 = n0 + wn * WN + l32;
+  const bool nobias = g.bias_mode == 0;
+  float* __restrict__ Wp =
+      g.ws ? g.ws + blockIdx.y * g.M * g.N : nullptr;
+  // the general case of one element: its sum a at (row, col)
+  auto finish = [&](int64_t row, int64_t col, float a) {
+    if (Wp) {
+      Wp[row * g.N + col] = a;
+      return;
+    }
+    float v = g.alpha * a;
+    float* cp = C + row * g.ldc + col;
+    if (g.beta != 0.f) v += g.beta * *cp;
+    if (g.bias_mode == 1) v += g.bias[col];
+    else if (g.bias_mode == 2) v += g.bias[row];
+    *cp = epilogue_act(g, row, col, v);
+  };
+  // An infinity or NaN among the operands (or a finite value that rounds to
+  // infinity in bfloat16) makes parts of the split NaN: a wave whose sums
+  // are not all finite forms them again from the floats themselves, with
+  // the infinities and NaNs of float arithmetic.  0 * x is 0 for finite x
+  // and NaN otherwise.
+  {
+    float z[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) z[r & 3] = __builtin_fmaf(acc[i][j][r], 0.f, z[r & 3]);
+    const float zz = (z[0] + z[1]) + (z[2] + z[3]);
+    if (__any(!(zz == 0.f))) {
+#pragma unroll 1
+      for (int e = 0; e < FM * FN * 16; ++e) {
+        const int r = e & 15, ij = e >> 4;
+        const int64_t row = r0 + (ij / FN) * 32 + 8 * (r >> 2) + (r & 3), col = c0 + (ij % FN) * 32;
+        if (EDGE && (row >= g.M || col >= g.N)) continue;
+        float s = 0.f;
+#pragma unroll 1
+        for (int64_t k = kbeg; k < kend; ++k) {
+          const float a = TA ? A[k * g.lda + row] : A[row * g.lda + k];
+          s = __builtin_fmaf(a, TB ? B[col * g.ldb + k] : B[k * g.ldb + col], s);
+        }
+        finish(row, col, s);
+      }
+      return;
+    }
+  }
+  // the sign of this lane's column after the last K tile; odd rows carry the
+  // other one
+  const int64_t kt = kend > kbeg ? cdiv(kend - kbeg, BK) : 1;
+  const float sign = (l32 + (kt - 1) / kFlip) & 1 ? -1.f : 1.f, alpha = g.alpha * sign;
+  auto each = [&](auto&& put) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        if (EDGE && c0 + j * 32 >= g.N) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int ro = i * 32 + 8 * (r >> 2) + (r & 3);
+          if (!EDGE || r0 + ro < g.M) put(r & 1 ? -acc[i][j][r] : acc[i][j][r], ro, j * 32);
+        }
+      }
+  };
+  if (Wp) {
+    // raw partial sums; the reduce kernel applies alpha / beta / bias
+    float* __restrict__ W = Wp + r0 * g.N + c0;
+    const int64_t ld = g.N;
+    each([&](float a, int ro, int co) { W[ro * ld + co] = sign * a; });
+    return;
+  }
+  float* __restrict__ Cb = C + r0 * g.ldc + c0;
+  const int64_t ldc = g.ldc, ldx = g.ldaux;
+  float* __restrict__ Xb = g.aux ? g.aux + r0 * ldx + c0 : nullptr;
+  if (g.beta == 0.f && nobias && g.act == 0) {
+    each([&](float a, int ro, int co) { Cb[ro * ldc + co] = alpha * a; });
+    return;
+  }
+  if (g.beta == 0.f && g.bias_mode == 1 && (g.act == 0 || g.act == 1 || g.act == 3)) {
+    // bias per column (+ GELU or + residual)
+    const float* __restrict__ bb = g.bias + c0;
+    const int act = g.act;
+    auto run = [&](auto ACT) {
+      constexpr int A_ = decltype(ACT)::value;
+      each([&](float a, int ro, int co) {
+        float v = alpha * a + bb[co];
+        if (A_ == 1) {
+          v = gelu_f(v);
+        } else if (A_ == 3) {
+          v += Xb[ro * ldx + co];
+        }
+        Cb[ro * ldc + co] = v;
+      });
+    };
+    if (act == 0) run(IConst<0>());
+    else if (act == 1) run(IConst<1>());
+    else run(IConst<3>());
+  } else {
+    each([&](float a, int ro, int co) { finish(r0 + ro, c0 + co, sign * a); });
+  }
+}
+
+struct TileCfg {
+  int bm, bn, wr, wc;  // block tile, wave rows and columns
+};
+constexpr TileCfg kTiles[] = {{256, 256, 2, 4}, {256, 192, 4, 2}, {256, 128, 2, 2},
+                              {128, 128, 2, 2}, {128, 64, 2, 2},  {64, 64, 2, 2}};
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+
+template <int BM, int BN, int WR, int WC, bool EDGE>
+void launch_split_e(const GemmArgs& g, dim3 grid, int ta, int tb) {
+  const dim3 block(WR * WC * 64);
+  if (!ta && !tb)
+    tjh_launch((k_gemm_split<BM, BN, WR, WC, false, false, EDGE>), grid, block, 0, stream(), g);
+  else if (!ta && tb)
+    tjh_launch((k_gemm_split<BM, BN, WR, WC, false, true, EDGE>), grid, block, 0, stream(), g);
+  else
+    tjh_launch((k_gemm_split<BM, BN, WR, WC, true, false, EDGE>), grid, block, 0, stream(), g);
+}
+
+// One launch of tile I.  Each tile's kernels are compiled in a source file
+// of their own (gemm_split_*.hip).
+template <int I>
+void launch_split(const GemmArgs& g, dim3 grid, int ta, int tb, bool edge) {
+  constexpr TileCfg t = kTiles[I];
+  if (edge) launch_split_e<t.bm, t.bn, t.wr, t.wc, true>(g, grid, ta, tb);
+  else launch_split_e<t.bm, t.bn, t.wr, t.wc, false>(g, grid, ta, tb);
+}
+
+}  // namespace tjh
+
+/* tjh_gemm (batch 1) for a result that no gradient is taken through: float
+ * products formed from three bf16 parts of each operand.  Its error against
+ * 64 bits is under tjh_gemm's, but its roundings are others.  (Elements under
+ * 2^-109 in magnitude keep an absolute error of up to 2^-134.)
+ * act 0: nothing; 1: C = GELU(v); 3: C = residual + v, with residual [M][N]
+ * at row stride ldr, not overlapping C.  bias_mode 0, 1 or 2 as tjh_gemm.
+ * For the Python host, which knows what is recorded; not part of the
+ * library's declared interface. */
+extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,
+                              const float* A, int64_t lda, const float* B, int64_t ldb, float beta,
+                              float* C, int64_t ldc, const float* bias, int bias_mode,
+                              const float* residual, int64_t ldr, int act);

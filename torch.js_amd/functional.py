@@ -494,7 +494,8 @@ def linear(x, weight, bias=None):
     x2 = reshape(x.detach(), (M, in_f))
     wd = weight.detach()
     bd = bias.detach().contiguous() if bias is not None else None
-    out2 = _gemm(x2, wd.T, bias=bd, bias_mode=1 if bd is not None else 0)
+    out2 = _gemm(x2, wd.T, bias=bd, bias_mode=1 if bd is not None else 0,
+                 recorded=_T._recorded(x, weight, bias))
     out = reshape_raw(out2, lead + (out_f,))
     rx, rw = x.requires_grad, weight.requires_grad
     rb = bias is not None and bias.requires_grad
@@ -553,7 +554,8 @@ def _linear_add(x, weight, bias, residual):
     r2 = reshape(r if r.dtype == "float32" and r.is_contiguous() else r.float().contiguous(),
                  (M, out_f))
     out2 = empty((M, out_f))
-    _gemm(x2, wd.T, out=out2, bias=bd, bias_mode=1 if bd is not None else 0, aux=r2, act=3)
+    _gemm(x2, wd.T, out=out2, bias=bd, bias_mode=1 if bd is not None else 0, aux=r2, act=3,
+          recorded=_T._recorded(x, weight, bias, residual))
     out = reshape_raw(out2, lead + (out_f,))
     rx, rw = x.requires_grad, weight.requires_grad
     rb = bias is not None and bias.requires_grad
@@ -600,17 +602,20 @@ def _mlp_gelu(x, w1, b1, w2, b2, residual=None):
     if residual is not None and residual.shape != lead + (d_out,):
         raise RuntimeError("mlp: residual shape %s != output shape %s"
                            % (list(residual.shape), list(lead + (d_out,))))
-    h = empty((M, hid))
+    rec = _T._recorded(x, w1, b1, w2, b2, residual)
+    h = empty((M, hid)) if rec else None
     a = empty((M, hid))
-    _gemm(x2, w1d.T, out=a, bias=b1d, bias_mode=1 if b1d is not None else 0, aux=h, act=1)
+    _gemm(x2, w1d.T, out=a, bias=b1d, bias_mode=1 if b1d is not None else 0, aux=h, act=1,
+          recorded=rec)
     if residual is None:
-        y2 = _gemm(a, w2d.T, bias=b2d, bias_mode=1 if b2d is not None else 0)
+        y2 = _gemm(a, w2d.T, bias=b2d, bias_mode=1 if b2d is not None else 0, recorded=rec)
     else:
         r = residual.detach()
         r2 = reshape(r if r.dtype == "float32" and r.is_contiguous() else r.float().contiguous(),
                      (M, d_out))
         y2 = empty((M, d_out))
-        _gemm(a, w2d.T, out=y2, bias=b2d, bias_mode=1 if b2d is not None else 0, aux=r2, act=3)
+        _gemm(a, w2d.T, out=y2, bias=b2d, bias_mode=1 if b2d is not None else 0, aux=r2, act=3,
+              recorded=rec)
     out = reshape_raw(y2, lead + (d_out,))
     need = [t is not None and t.requires_grad for t in (x, w1, b1, w2, b2)]
 

@@ -2762,15 +2762,22 @@ def _mat_operand(t):
     return None
 
 
+def _recorded(*ts):
+    """Whether an op on these tensors records a graph node."""
+    return _grad["enabled"] and any(t is not None and t.requires_grad for t in ts)
+
+
 def _gemm(a, b, out=None, alpha=1.0, beta=0.0, bias=None, bias_mode=0, rowsum_out=None,
-          aux=None, act=0):
+          aux=None, act=0, recorded=True):
     """out[M,N] = alpha*a[M,K] @ b[K,N] (+beta*out) (+bias) for 2-D views.
     rowsum_out (a contiguous [M] tensor) receives the row sums of `a` from
     the same launch (bias_mode 3: a Linear layer's bias gradient computed
     with its weight gradient).  act 1 / 2 / 3 with aux ([M,N], row stride
     as out's) fuses an elementwise op into the epilogue: 1 writes the
     pre-activation to aux and GELU of it to out, 2 multiplies by
-    GELU'(aux), 3 adds aux (a residual; must not overlap out)."""
+    GELU'(aux), 3 adds aux (a residual; must not overlap out).  recorded
+    False (no gradient is taken through the result): split products, and
+    act 1 keeps no pre-activation."""
     if rowsum_out is not None:
         assert bias is None and bias_mode == 0 and rowsum_out.is_contiguous()
         bias, bias_mode = rowsum_out, 3
@@ -2788,6 +2795,13 @@ def _gemm(a, b, out=None, alpha=1.0, beta=0.0, bias=None, bias_mode=0, rowsum_ou
     if out is None:
         out = _empty_padded(M, N) if N % 4 else empty((M, N))
     ldc = out._strides[0] if out._strides[0] >= N else N
+    if not recorded:
+        L.check(L.lib().tjh_gemm_split(1 if oa[2] else 0, 1 if ob[2] else 0, M, N, K, float(alpha),
+                                       oa[0], oa[1], ob[0], ob[1], float(beta), out.data_ptr(),
+                                       ldc, bias.data_ptr() if bias is not None else None,
+                                       bias_mode, aux.data_ptr() if act == 3 else None,
+                                       aux._strides[0] if act == 3 else 0, act), "gemm_split")
+        return out
     if act:
         assert aux is not None and aux.shape == (M, N) and aux._strides[1] == 1
         L.check(L.lib().tjh_gemm_act(1 if oa[2] else 0, 1 if ob[2] else 0, M, N, K, float(alpha),
@@ -2918,7 +2932,7 @@ def matmul(a, b):
 
 
 def _mm(a, b):
-    out = _gemm(a, b)
+    out = _gemm(a, b, recorded=_recorded(a, b))
 
     def bwd(g):
         ga = _gemm(g, b.detach().T) if a.requires_grad else None
