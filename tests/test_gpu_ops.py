@@ -987,6 +987,28 @@ def test_gemm_split_error_of_scaled_operands(torch, scale):
     assert np.linalg.norm(got - want) <= 4.8e-7 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 7, 8, 9])
+@pytest.mark.parametrize("N,K,shift", [(1, 33, 0), (770, 768, 0), (2049, 1001, 1), (8200, 40, 2),
+                                       (65, 3071, 3)])
+def test_few_rows_products(torch, M, N, K, shift):
+    """Up to 8 rows times a transposed matrix: one or four columns a wave,
+    the waves sharing a column's K, K tails and odd alignment, and the 9
+    rows that go to the tiles."""
+    r = np.random.default_rng(M * N + K)
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    bias, res, C0 = (f32(r.standard_normal(n)) for n in (N, (M, N), (M, N)))
+    bm, BT = f32(r.standard_normal(M)), np.ascontiguousarray(B.T)
+    z, z32 = A.astype(np.float64) @ B.astype(np.float64), A @ B
+
+    def raw(**k):
+        return _raw_split(torch, 0, 1, A, BT, M, N, K, shift=shift, **k)
+    check_floor(raw(alpha=0.5, beta=0.25, C0=C0, bias=bias, bmode=1), 0.5 * z + 0.25 * C0 + bias,
+                np.float32(0.5) * z32 + np.float32(0.25) * C0 + bias)
+    check_floor(raw(bias=bm, bmode=2, res=res, act=3), z + bm[:, None] + res, z32 + bm[:, None] + res)
+    s = 1 / np.sqrt(K)
+    check(raw(alpha=s, bias=bias, bmode=1, act=1), ops.unary("gelu", s * z + bias), **RED)
+
+
 def test_products_without_gradient_take_the_split_kernels(torch):
     """Linear, the residual and MLP forms and matmul: split products exactly
     where nothing is recorded, equal to the recorded ones within rounding."""

@@ -2,6 +2,7 @@
 // split-K and the C entry point.
 
 #include "gemm_split.h"
+#include "gemm_rows.h"
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -151,6 +152,9 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   g.ldaux = ldr;
   g.act = act;
   KernelScope ks("gemm");
+  // few rows: nothing to gain from the matrix cores
+  if (!transA && transB && M <= kFewRows && g.vecA && g.vecB && cdiv(N, 4) < (int64_t(1) << 31))
+    return gemm_rows(g, cus);
   const Plan plan = choose_plan(M, N, K, cus);
   const TileCfg& tc = kTiles[plan.tile];
   g.tiles_m = (int)cdiv(M, tc.bm);
