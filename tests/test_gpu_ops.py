@@ -1009,6 +1009,53 @@ def test_few_rows_products(torch, M, N, K, shift):
     check(raw(alpha=s, bias=bias, bmode=1, act=1), ops.unary("gelu", s * z + bias), **RED)
 
 
+def _attend64(q, k, v, causal):
+    q, k, v = (a.astype(np.float64) for a in (q, k, v))
+    s = q @ k.swapaxes(-1, -2) / np.sqrt(q.shape[-1])
+    if causal:
+        s = np.where(np.tril(np.ones(s.shape[-2:], bool)), s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    return (p / p.sum(-1, keepdims=True)) @ v
+
+
+@pytest.mark.parametrize("D", [4, 40, 64, 80, 128])
+@pytest.mark.parametrize("Tq,Tk,causal", [(1, 1, False), (1, 63, False), (1, 257, False),
+                                          (1, 701, True), (1, 1025, False), (2, 900, False),
+                                          (129, 129, True), (333, 333, True), (300, 130, False),
+                                          (512, 512, True)])
+def test_attention_of_few_workgroups(torch, D, Tq, Tk, causal):
+    """One query over a workgroup, and queries split over their keys where
+    no gradient is recorded, from a cache longer than the keys: partial
+    tiles, slices past a causal block's end, the padded head dims."""
+    r = np.random.default_rng(Tq + Tk + D)
+    B, H = 2, 3
+    q = f32(r.standard_normal((B, H, Tq, D)))
+    k, v = (f32(r.standard_normal((B, H, Tk + 5, D))) for _ in range(2))
+    with torch.no_grad():
+        tk, tv = (torch.tensor(a)[:, :, :Tk] for a in (k, v))
+        got = torch.functional.scaled_dot_product_attention(torch.tensor(q), tk, tv,
+                                                            is_causal=causal).numpy()
+    # the recorded form: one workgroup for all keys of 128 queries
+    tq = torch.tensor(q, requires_grad=True)
+    rec = torch.functional.scaled_dot_product_attention(tq, tk, tv, is_causal=causal).detach().numpy()
+    want = _attend64(q, k[:, :, :Tk], v[:, :, :Tk], causal)
+    check(got, want, **RED)
+    assert np.linalg.norm(got - want) <= 1.5 * np.linalg.norm(rec - want) + 1e-7 * np.linalg.norm(want)
+
+
+def test_attention_key_split_of_large_and_masked_scores(torch):
+    """Scores of +-1e4 spread over the slices, and rows whose later slices
+    underflow against the first."""
+    r = np.random.default_rng(3)
+    q, k, v = (f32(r.standard_normal((1, 2, 260, 32))) for _ in range(3))
+    k[:, :, ::50] *= 3000
+    with torch.no_grad():
+        got = torch.functional.scaled_dot_product_attention(
+            *(torch.tensor(a) for a in (q, k, v)), is_causal=True).numpy()
+    # scores of 1e4 carry an absolute rounding error of 1e4 * 2^-23
+    check(got, _attend64(q, k, v, True), rtol=2e-2, atol=2e-2)
+
+
 def test_products_without_gradient_take_the_split_kernels(torch):
     """Linear, the residual and MLP forms and matmul: split products exactly
     where nothing is recorded, equal to the recorded ones within rounding."""

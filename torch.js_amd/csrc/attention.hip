@@ -21,6 +21,12 @@
 #include <float.h>
 
 namespace tjh {
+
+// attn_one.hip
+int attn_one_query(const float* q, const float* k, const float* v, float* o, float* lse, int64_t B,
+                   int64_t H, int64_t Tk, int64_t D, const int64_t* qs, const int64_t* ks,
+                   const int64_t* vs, const int64_t* os, float scale, int causal);
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -114,11 +120,18 @@ int tjh_sdpa_forward(const float* q, const float* k, const float* v, float* o, f
   {
     const void* ptrs[4] = {q, k, v, o};
     const int64_t* sts[4] = {qs, ks, vs, os};
-    if (flash_supported(D, ptrs, sts, 4))
+    const bool flash = flash_supported(D, ptrs, sts, 4);
+    // one query: its keys over a whole workgroup (701 keys, 48 heads: the
+    // flash kernel's chain of key tiles takes 58 us)
+    if (flash && Tq == 1)
+      return attn_one_query(q, k, v, o, lse, B, H, Tk, D, qs, ks, vs, os, scale, causal);
+    if (flash)
       return flash_forward(q, k, v, o, lse, B, H, Tq, Tk, D, qs, ks, vs, os, scale, causal);
   }
+  Scratch own_lse(lse ? 0 : (size_t)(B * H * Tq) * sizeof(float));
+  if (!lse) lse = own_lse.as<float>();
   Scratch S((size_t)(H * Tq * Tk) * sizeof(float));
-  if (!S.ok()) return set_error(TJH_ERR_OOM, "sdpa_forward: no scratch for scores");
+  if (!S.ok() || !lse) return set_error(TJH_ERR_OOM, "sdpa_forward: no scratch for scores");
   float* s = S.as<float>();
   KernelScope kscope("sdpa_fwd_composite");
   for (int64_t b = 0; b < B; ++b) {

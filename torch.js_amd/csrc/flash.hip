@@ -109,6 +109,12 @@ struct FlashArgs {
   float* dsblk;
   int nqt, nkt;       // 32-row query / key tiles per (b, h)
   int64_t spare_blk;  // index of the spare block after the last one
+  // key-split forward (no lse is wanted): slices of `kslice` key tiles, at
+  // most `nsl` for a query; part holds [slice][b*H + h][Tq][D] unscaled
+  // sums, pml [slice][b*H + h][Tq] {maximum, sum of exponentials}
+  float* part;
+  float2* pml;
+  int kslice, nsl;
 };
 
 // Column of key offset ko (0..31) inside a dS block row: the query-block
@@ -285,8 +291,9 @@ __device__ __forceinline__ void zero_acc(floatx16 (&acc)[NC]) {
 // ------------------------------------------------------------ forward
 
 // GUARD: Tk is not a multiple of 32 (the last key tile is partial), or D <
-// HD (padded columns).
-template <int HD, bool GUARD>
+// HD (padded columns).  PART: this workgroup takes one slice of the keys and
+// writes its running sums, which k_flash_merge adds up.
+template <int HD, bool GUARD, bool PART>
 __global__ __launch_bounds__(256, occ_fwd<HD>()) void k_flash_fwd(FlashArgs a) {
   using S_ = Hd<HD>;
   __shared__ __attribute__((aligned(16))) float Ks[2][TILE * S_::W];
@@ -302,6 +309,7 @@ __global__ __launch_bounds__(256, occ_fwd<HD>()) void k_flash_fwd(FlashArgs a) {
   const float* K = a.k + b * a.ks.b + hh * a.ks.h;
   const float* V = a.v + b * a.vs.b + hh * a.vs.h;
   const int q0 = qb * ROWS + w * TILE;  // this wave's first query
+  const int kb0 = PART ? (int)blockIdx.y * a.kslice : 0;  // first key tile
   const int myq = q0 + l32;
 
   float qf[S_::RUN];
@@ -312,15 +320,19 @@ __global__ __launch_bounds__(256, occ_fwd<HD>()) void k_flash_fwd(FlashArgs a) {
 
   int kend = a.Tk;
   if (a.causal) kend = min(kend, qb * ROWS + ROWS);
-  const int nkb = (kend + TILE - 1) / TILE;
+  int nkb = (kend + TILE - 1) / TILE;
+  if (PART) {
+    if (kb0 >= nkb) return;  // this block's keys end before the slice
+    nkb = min(nkb, kb0 + a.kslice);
+  }
   floatx4 rk[S_::NC], rv[S_::NC];
-  load_tile<HD, GUARD>(K, a.ks.t, 0, a.Tk, a.D, rk);
-  load_tile<HD, GUARD>(V, a.vs.t, 0, a.Tk, a.D, rv);
+  load_tile<HD, GUARD>(K, a.ks.t, kb0 * TILE, a.Tk, a.D, rk);
+  load_tile<HD, GUARD>(V, a.vs.t, kb0 * TILE, a.Tk, a.D, rv);
   store_tile<HD>(Ks[0], rk);
   store_tile<HD>(Vs[0], rv);
   __syncthreads();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int cur = kb & 1;
+  for (int kb = kb0; kb < nkb; ++kb) {
+    const int cur = (kb - kb0) & 1;
     const bool more = kb + 1 < nkb;
     if (more) {
       load_tile<HD, GUARD>(K, a.ks.t, (kb + 1) * TILE, a.Tk, a.D, rk);
@@ -372,12 +384,49 @@ __global__ __launch_bounds__(256, occ_fwd<HD>()) void k_flash_fwd(FlashArgs a) {
     }
     __syncthreads();
   }
+  if constexpr (PART) {
+    const int64_t row0 = ((int64_t)blockIdx.y * nbh + bh) * a.Tq;
+    write_rows<HD>(w < 2 ? Ks[w] : Vs[w - 2], acc, 1.0f, a.part + row0 * a.D, a.D, q0, a.Tq, a.D,
+                   l32, h, lane);
+    if (h == 0 && myq < a.Tq) a.pml[row0 + myq] = make_float2(m, lsum);
+    return;
+  }
   // every accumulator of a lane belongs to its query column: scale by 1/l
   const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
   float* obase = a.out + b * a.os.b + hh * a.os.h;
   float* buf = (w < 2 ? Ks[w] : Vs[w - 2]);
   write_rows<HD>(buf, acc, inv, obase, a.os.t, q0, a.Tq, a.D, l32, h, lane);
   if (h == 0 && myq < a.Tq) a.lse_out[bh * a.Tq + myq] = (m + __log2f(lsum)) * kLn2;
+}
+
+// The slices of the key-split forward: o = (sum of 2^(m_s - m) acc_s) /
+// (sum of 2^(m_s - m) l_s), in the order of the slices.  One float4 a lane.
+__global__ __launch_bounds__(256) void k_flash_merge(FlashArgs a, int64_t n4) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const int d4 = a.D / 4;
+  const int64_t row = i / d4, rows = n4 / d4;  // row: (b * H + h) * Tq + q
+  const int c = (int)(i - row * d4);
+  const int64_t bh = row / a.Tq;
+  const int q = (int)(row - bh * a.Tq);
+  // slices of this query's block of ROWS (the ones that were written)
+  const int kend = a.causal ? min(a.Tk, q / ROWS * ROWS + ROWS) : a.Tk;
+  const int n = ((kend + TILE - 1) / TILE + a.kslice - 1) / a.kslice;
+  float top = -INFINITY;
+  for (int s = 0; s < n; ++s) top = fmaxf(top, a.pml[s * rows + row].x);
+  const float ts = top == -INFINITY ? 0.f : top;
+  floatx4 o = {0.f, 0.f, 0.f, 0.f};
+  float den = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < n; ++s) {
+    const float2 ml = a.pml[s * rows + row];
+    const float f = exp2_hw(ml.x - ts);
+    den = __builtin_fmaf(ml.y, f, den);
+    o += f * *reinterpret_cast<const floatx4*>(a.part + (s * rows + row) * a.D + 4 * c);
+  }
+  const int64_t b = bh / a.H, h = bh % a.H;
+  *reinterpret_cast<floatx4*>(a.out + b * a.os.b + h * a.os.h + q * a.os.t + 4 * c) =
+      o * (den > 0.f ? 1.0f / den : 0.f);
 }
 
 // ------------------------------------------------------------ backward
@@ -921,10 +970,34 @@ int padded_hd(int64_t D) { return (int)((D + 31) / 32 * 32); }
 
 template <int HD>
 void launch_forward(const FlashArgs& a, unsigned grid) {
-  if ((a.Tk % TILE) || a.D != HD)
-    tjh_launch(k_flash_fwd<HD, true>, dim3(grid), dim3(256), 0, stream(), a);
+  const bool guard = (a.Tk % TILE) || a.D != HD;
+  if (a.part && guard)
+    tjh_launch(k_flash_fwd<HD, true, true>, dim3(grid, a.nsl), dim3(256), 0, stream(), a);
+  else if (a.part)
+    tjh_launch(k_flash_fwd<HD, false, true>, dim3(grid, a.nsl), dim3(256), 0, stream(), a);
+  else if (guard)
+    tjh_launch(k_flash_fwd<HD, true, false>, dim3(grid), dim3(256), 0, stream(), a);
   else
-    tjh_launch(k_flash_fwd<HD, false>, dim3(grid), dim3(256), 0, stream(), a);
+    tjh_launch(k_flash_fwd<HD, false, false>, dim3(grid), dim3(256), 0, stream(), a);
+}
+
+// Key tiles per slice of a forward pass of BH heads, or 0 where its blocks
+// of ROWS queries fill the CUs by themselves.  A block walks its key tiles
+// one after the other, 2.6 us each, on one CU: 12 heads of 777 queries are 84
+// workgroups, the longest of 25 tiles.  Slices of at least 4 tiles (fewer
+// spend as long on their prologue and on the merge) that make two workgroups
+// a CU: 27 + 6 us, 65 unsplit.
+int key_slice(int64_t BH, int64_t Tq, int64_t Tk, int causal) {
+  const int64_t cus = num_cus() > 0 ? num_cus() : 256, blocks = cdiv(Tq, ROWS);
+  const int64_t nkt = cdiv(Tk, TILE);
+  if (BH * blocks >= cus || nkt <= 4) return 0;
+  int64_t tiles = 0;
+  for (int64_t i = 0; i < blocks; ++i) {
+    const int64_t end = (i + 1) * (ROWS / TILE);
+    tiles += causal && end < nkt ? end : nkt;
+  }
+  const int64_t s = cdiv(tiles * BH, 2 * cus);
+  return (int)(s < 4 ? 4 : s);
 }
 
 // The key kernel (dK, dV) then the query kernel (dQ) of the backward; a.out
@@ -991,6 +1064,19 @@ int flash_forward(const float* q, const float* k, const float* v, float* o, floa
   a.cus = cus_per_xcd();
   const int64_t grid = B * H * a.nblk;
   TJH_ARG(grid < (int64_t(1) << 31), "sdpa: grid too large");
+  // slices of the keys only without lse: a recorded pass keeps its roundings
+  const int64_t rows = B * H * Tq;
+  a.kslice = lse ? 0 : key_slice(B * H, Tq, Tk, causal);
+  a.nsl = a.kslice ? (int)cdiv(cdiv(Tk, TILE), a.kslice) : 1;
+  Scratch part(a.nsl > 1 ? (size_t)(a.nsl * rows * (D + 2)) * sizeof(float) : 0);
+  Scratch own_lse(!lse && !part.ok() ? (size_t)rows * sizeof(float) : 0);
+  if (part.ok()) {
+    a.part = part.as<float>();
+    a.pml = reinterpret_cast<float2*>(a.part + a.nsl * rows * D);
+  } else if (!lse) {  // one slice, or no scratch for more
+    if (!own_lse.ok()) return set_error(TJH_ERR_OOM, "sdpa_forward: no scratch");
+    a.lse_out = own_lse.as<float>();
+  }
   KernelScope ks_("sdpa_fwd");
   switch (padded_hd(D)) {
     case 32: launch_forward<32>(a, (unsigned)grid); break;
@@ -998,7 +1084,12 @@ int flash_forward(const float* q, const float* k, const float* v, float* o, floa
     case 96: launch_forward<96>(a, (unsigned)grid); break;
     default: launch_forward<128>(a, (unsigned)grid); break;
   }
-  return check_launch("flash_forward");
+  const int rc = check_launch("flash_forward");
+  if (rc != TJH_OK || !a.part) return rc;
+  const int64_t n4 = rows * D / 4;
+  TJH_ARG(cdiv(n4, 256) < (int64_t(1) << 31), "sdpa: grid too large");
+  tjh_launch(k_flash_merge, dim3((unsigned)cdiv(n4, 256)), dim3(256), 0, stream(), a, n4);
+  return check_launch("flash_merge");
 }
 
 int flash_backward(const float* q, const float* k, const float* v, const float* o,
