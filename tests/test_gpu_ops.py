@@ -1056,6 +1056,55 @@ def test_attention_key_split_of_large_and_masked_scores(torch):
     check(got, _attend64(q, k, v, True), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("B,T,C,heads", [(1, 1, 64, 2), (2, 37, 96, 3), (3, 130, 160, 2)])
+def test_block_without_gradient_is_one_call(torch, monkeypatch, B, T, C, heads):
+    """Block under no_grad, plain and cached, gives bit for bit what its
+    layers give one by one, and leaves the same cache; with a layer or a
+    forward of another kind, or without biases, it takes the layers."""
+    from torchjs_amd import workloads as W
+    torch.manual_seed(5)
+    blk = W.Block(C, heads)
+    x = torch.tensor(f32(np.random.default_rng(1).standard_normal((B, T, C))))
+    y = torch.tensor(f32(np.random.default_rng(2).standard_normal((B, 1, C))))
+    fast = W.Block._infer
+    calls = []
+    monkeypatch.setattr(W.Block, "_infer",
+                        lambda self, *a: calls.append(fast(self, *a)) or calls[-1])
+
+    def run():
+        with torch.no_grad():
+            cache = W.KVCache(1, B, heads, T + 3, C // heads)
+            out = [blk(x), blk.forward_cached(x, cache, 0, 0), blk.forward_cached(y, cache, 0, T)]
+            return [a.numpy() for a in out + cache.k + cache.v]
+    got = run()
+    assert len(calls) == 3 and all(c is not None for c in calls)
+    with monkeypatch.context() as m:
+        m.setattr(W.Block, "_infer", lambda self, *a: None)
+        want = run()
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+    with torch.no_grad():
+        cache = W.KVCache(1, B, heads, T, C // heads)
+        with pytest.raises(RuntimeError):
+            blk.forward_cached(y, cache, 0, T)  # beyond the cache
+        del calls[:]
+        lin = blk.mlp.c_fc
+        blk.mlp.c_fc = torch.nn.Linear(C, 4 * C, bias=False)
+        blk(x)
+        assert calls[-1] is not None  # a missing bias is still one call
+        blk.mlp.c_fc = type("Mine", (torch.nn.Linear,), {})(C, 4 * C)
+        blk(x)
+        assert calls[-1] is None
+        blk.mlp.c_fc = lin
+        blk.attn.forward = lambda h, residual=None: residual
+        blk(x)
+        assert calls[-1] is None
+    del blk.attn.__dict__["forward"]
+    n = len(calls)
+    blk(x).sum().backward()
+    assert len(calls) == n
+
+
 def test_products_without_gradient_take_the_split_kernels(torch):
     """Linear, the residual and MLP forms and matmul: split products exactly
     where nothing is recorded, equal to the recorded ones within rounding."""
@@ -1077,7 +1126,8 @@ def test_products_without_gradient_take_the_split_kernels(torch):
         y = blk(x).numpy()
         assert not calls
         with torch.no_grad():
-            z = blk(x).numpy()
+            z = blk.attn(blk.ln_1(x), residual=x)
+            z = blk.mlp(blk.ln_2(z), residual=z).numpy()
             (x.reshape(80, 64) @ x.reshape(80, 64).t()).numpy()
     finally:
         L._lib = real_lib

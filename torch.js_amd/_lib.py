@@ -171,6 +171,8 @@ SIGNATURES = {
                      c_vp, c_i64, c_vp, c_int, c_vp, c_i64, c_int],
     "tjh_gemm_split": [c_int, c_int, c_i64, c_i64, c_i64, c_f32, c_vp, c_i64, c_vp, c_i64, c_f32,
                        c_vp, c_i64, c_vp, c_int, c_vp, c_i64, c_int],
+    "tjh_block_infer": [c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_f32, c_f32,
+                        c_vp, c_vp, c_i64, c_i64],
     "tjh_gemm_ce": [c_int, c_i64, c_i64, c_i64, c_vp, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp,
                     c_i64],
     "tjh_sdpa_forward": [c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, P_i64,

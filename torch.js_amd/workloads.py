@@ -9,9 +9,13 @@ user would write it (nn modules, functional ops, backward(), optimizers):
   * Block   pre-LN transformer block (causal SDPA, 4x GELU MLP)
   * GPT2    GPT-2 small with tied embeddings, next-token cross_entropy
 """
+import ctypes
+import math
+
+from . import _lib as L
 from . import functional as F
 from . import nn
-from .tensor import arange, from_numpy, no_grad, zeros
+from .tensor import (_before_write, arange, empty, from_numpy, is_grad_enabled, no_grad, zeros)
 
 
 def mlp():
@@ -127,12 +131,85 @@ class Block(nn.Module):
 
     def forward(self, x):
         # x + attn(ln_1(x)), then x + mlp(ln_2(x))
+        if not is_grad_enabled():
+            y = self._infer(x)
+            if y is not None:
+                return y
         x = self.attn(self.ln_1(x), residual=x)
         return self.mlp(self.ln_2(x), residual=x)
 
+    def _infer(self, x, cache=None, layer=0, pos=0):
+        """The block as one library call that issues the same launches (a
+        decoding step's eight take 225 us of host time one by one), where no
+        graph is recorded and the block is made of the plain layers in
+        float32; None anywhere else."""
+        at, mlp = self.attn, self.mlp
+        if type(at) is not CausalSelfAttention or type(mlp) is not MLPBlock:
+            return None
+        mods = (self.ln_1, at, at.c_attn, at.c_proj, self.ln_2, mlp, mlp.c_fc, mlp.c_proj)
+        if not (tuple(map(type, mods)) == _BLOCK_MODULES and at.fused and mlp.fused and
+                x.ndim == 3 and x.dtype == "float32"):
+            return None
+        if any("forward" in m.__dict__ or "forward_cached" in m.__dict__ for m in mods):
+            return None
+        B, T, C = x.shape
+        hd, hid = C // at.heads, mlp.c_fc.weight.shape[0]
+        ln = ((C,), (C,))
+        if not (x.numel() and C == at.d and C % at.heads == 0 and hd % 4 == 0 and
+                hid % 4 == 0 and self.ln_1.normalized_shape == (C,) and
+                self.ln_2.normalized_shape == (C,) and x.is_contiguous()):
+            return None
+        w = []
+        for m, shapes in ((mods[0], ln), (mods[2], ((3 * C, C), (3 * C,))),
+                          (mods[3], ((C, C), (C,))), (mods[4], ln),
+                          (mods[6], ((hid, C), (hid,))), (mods[7], ((C, hid), (C,)))):
+            for t, shape in zip((m.weight, m.bias), shapes):
+                if t is None:  # a bias, or a norm without weights
+                    w.append(None)
+                    continue
+                if t.shape != shape or t.dtype != "float32" or not t.is_contiguous():
+                    return None
+                w.append(t.data_ptr())
+        kc = vc = None
+        max_len = 0
+        if cache is not None:
+            if type(cache) is not KVCache or pos < 0 or (pos and T != 1):
+                return None
+            kc, vc = cache.k[layer], cache.v[layer]
+            max_len = cache.max_len
+            for t in (kc, vc):
+                if t.shape != (B, at.heads, max_len, hd) or t.dtype != "float32" or \
+                        not t.is_contiguous() or t.requires_grad:
+                    return None
+            if pos + T > max_len:
+                return None
+        px = x.data_ptr()
+        ptrs = w + [px] if cache is None else w + [px, kc.data_ptr(), vc.data_ptr()]
+        if any(p is not None and p & 15 for p in ptrs):
+            return None
+        if cache is not None:
+            _before_write(kc, vc)
+        y = empty((B, T, C))
+        L.check(L.lib().tjh_block_infer(
+            px, y.data_ptr(), (ctypes.c_void_p * 12)(*w), B, T, C, at.heads, hid,
+            float(self.ln_1.eps), float(self.ln_2.eps), 1.0 / math.sqrt(hd),
+            kc.data_ptr() if kc is not None else None, vc.data_ptr() if vc is not None else None,
+            max_len, pos), "block_infer")
+        return y
+
     def forward_cached(self, x, cache, layer, pos):
+        if not is_grad_enabled():
+            y = self._infer(x, cache, layer, pos)
+            if y is not None:
+                return y
         x = self.attn.forward_cached(self.ln_1(x), cache, layer, pos, residual=x)
         return self.mlp(self.ln_2(x), residual=x)
+
+
+# the layers of a block that _infer stands for: ln_1, attn, its two
+# projections, ln_2, mlp, its two layers
+_BLOCK_MODULES = (nn.LayerNorm, CausalSelfAttention, nn.Linear, nn.Linear, nn.LayerNorm, MLPBlock,
+                  nn.Linear, nn.Linear)
 
 
 class KVCache:
