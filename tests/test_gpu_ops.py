@@ -928,6 +928,30 @@ def test_gemm_split_epilogues(torch, M, N, K):
 
 
 @pytest.mark.parametrize("tile", SPLIT_TILES)
+@pytest.mark.parametrize("ta,M,N,K,shift", [(1, 512, 384, 64, 0), (1, 300, 5, 4000, 0),
+                                            (1, 257, 300, 541, 1), (1, 70, 3, 31, 0),
+                                            (0, 90, 70, 1, 0), (0, 90, 70, 200, 0)])
+def test_gemm_split_row_sums_every_tile(torch, monkeypatch, tile, ta, M, N, K, shift):
+    """A weight gradient with the row sums of op(A) beside it: whole tiles,
+    edges, K tails, slices of K, and what the float cores take (K < 32, A
+    stored [M][K], as the transpose of a gradient of one row is)."""
+    monkeypatch.setenv("TJH_SPLIT_TILE", tile)
+    r = np.random.default_rng(M + K)
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    from torchjs_amd import _lib as L
+    a, b = (torch.tensor(np.concatenate([np.zeros(shift, np.float32), x.ravel()]))
+            for x in (np.ascontiguousarray(A.T) if ta else A, B))
+    c, s = torch.zeros(M, N), torch.zeros(M)
+    L.check(L.lib().tjh_gemm_split(ta, 0, M, N, K, 1.0, a.data_ptr() + 4 * shift, M if ta else K,
+                                   b.data_ptr() + 4 * shift, N, 0.0, c.data_ptr(), N, s.data_ptr(),
+                                   3, None, 0, 0))
+    check_floor(c.numpy(), A.astype(np.float64) @ B.astype(np.float64), A @ B)
+    # the compensated sums of up to 64 slices, each within 4.5 sqrt(K) in
+    # magnitude, added one by one: about sqrt(64) roundings of half an ulp
+    assert np.abs(s.numpy() - A.astype(np.float64).sum(1)).max() <= 36 * 2 ** -24 * np.sqrt(K)
+
+
+@pytest.mark.parametrize("tile", SPLIT_TILES)
 @pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0)])
 def test_gemm_split_not_finite_every_tile(torch, monkeypatch, tile, ta, tb):
     """Infinities, NaNs and floats above the largest bfloat16 give the sums

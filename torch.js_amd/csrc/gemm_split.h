@@ -1,9 +1,10 @@
 // fp32 GEMM on the CDNA4 bf16 matrix cores: products of floats split into
 // three bf16 parts.  Serves the products that no gradient is taken through
-// (tjh_gemm_split); gemm.hip's float matrix cores serve the recorded ones,
-// whose roundings a training run depends on: AdamW's g / (|g| + eps)
-// amplifies any change of them to 2e-5 in the second step's gradients of
-// GPT-2, in which the float path itself is 1.6e-5 from 64 bits.
+// and large weight gradients (tjh_gemm_split); gemm.hip's float matrix cores
+// serve the other recorded ones, whose roundings a training run depends on:
+// AdamW's g / (|g| + eps) amplifies a change of all of them to 2e-5 in the
+// second step's gradients of GPT-2, in which the float path itself is
+// 1.6e-5 from 64 bits.
 //
 // Stands for matmul.wgsl:17-50 behind Tensor.matmul / mm and nn.Linear
 // (Tensor.ts:2132-2331, src/nn/linear.ts:43-66) under no_grad.
@@ -52,6 +53,7 @@
 #pragma once
 
 #include "gemm_args.h"
+#include "kahan.h"
 
 namespace tjh {
 
@@ -177,6 +179,18 @@ struct Tile {
       }
     }
   }
+  // Adds the tile's k values of each outer index to its running sum.
+  __device__ __forceinline__ void sum(Kahan (&s)[I][W]) const {
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      if (!has(i)) continue;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[i][w].add(r[i][w][k]);
+      }
+    }
+  }
   // Splits the tile and stores its parts in LDS, `part` bytes apart, outer
   // index o negated where o + flip is odd (kFlip below).
   __device__ __forceinline__ void store(char* __restrict__ S, int part, int flip) const {
@@ -289,6 +303,11 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   using TileB = Tile<TB, BN, T, EDGE>;
   TileA ta, ta2;
   TileB tb, tb2;
+  // bias_mode 3: the workgroups of the first column tile also sum the rows
+  // of op(A) over their K range (the bias gradient of a weight gradient),
+  // from the floats in flight to LDS
+  const bool row_sums = TA && g.bias_mode == 3 && tn == 0;
+  Kahan rsum[TileA::I][TileA::W];
   auto fetch = [&](int64_t t, TileA& xa, TileB& xb) {
     const int64_t k0 = kbeg + t * BK;
     xa.load(A, g.lda, g.M, m0, k0);
@@ -296,6 +315,7 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   };
   auto stage = [&](int64_t t, TileA& xa, TileB& xb) {
     char* S = lds + (t & 1) * BUF;
+    if (TA && row_sums) xa.sum(rsum);
     xa.store(S, PA, (int)(t / kFlip) & 1);
     xb.store(S + 3 * PA, PB, 0);
   };
@@ -389,6 +409,22 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   }
 
   __builtin_amdgcn_s_setprio(3);
+  if (TA && row_sums) {
+    // the two k halves of a row are in two lanes; the operand tiles are free
+    // here (the K loop ended on a barrier)
+    float(*rp)[BM] = reinterpret_cast<float(*)[BM]>(lds);
+#pragma unroll
+    for (int i = 0; i < TileA::I; ++i) {
+      if (!TileA::has(i)) continue;
+      int o, kq;
+      TileA::at(i, o, kq);
+#pragma unroll
+      for (int w = 0; w < TileA::W; ++w) rp[kq][o + w] = rsum[i][w].s;
+    }
+    __syncthreads();
+    for (int o = threadIdx.x; o < BM && m0 + o < g.M; o += T)
+      (g.rsw ? g.rsw + blockIdx.y * g.M : const_cast<float*>(g.bias))[m0 + o] = rp[0][o] + rp[1][o];
+  }
 
   // ---- epilogue
   // Element (i, j, r) of this wave sits at row r0 + ro(i, r), column
@@ -398,7 +434,7 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   // the epilogue runs beside the other workgroup's MFMAs, where every
   // vector instruction it issues is slow.
   const int64_t r0 = m0 + wm * WM + 4 * h, c0 = n0 + wn * WN + l32;
-  const bool nobias = g.bias_mode == 0;
+  const bool nobias = g.bias_mode == 0 || g.bias_mode == 3;
   float* __restrict__ Wp =
       g.ws ? g.ws + blockIdx.y * g.M * g.N : nullptr;
   // the general case of one element: its sum a at (row, col)
@@ -534,7 +570,8 @@ void launch_split(const GemmArgs& g, dim3 grid, int ta, int tb, bool edge) {
  * 64 bits is under tjh_gemm's, but its roundings are others.  (Elements under
  * 2^-109 in magnitude keep an absolute error of up to 2^-134.)
  * act 0: nothing; 1: C = GELU(v); 3: C = residual + v, with residual [M][N]
- * at row stride ldr, not overlapping C.  bias_mode 0, 1 or 2 as tjh_gemm.
+ * at row stride ldr, not overlapping C.  bias_mode 0 to 3 as tjh_gemm, 3
+ * (bias receives the row sums of op(A)) with act 0 only.
  * For the Python host, which knows what is recorded; not part of the
  * library's declared interface. */
 extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,

@@ -51,7 +51,12 @@ struct Plan {
 //
 // TJH_SPLIT_TILE=BMxBN forces a tile (read on every call, so a test can
 // sweep the tiles in one process).
-Plan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
+//
+// With A transposed (a weight gradient, K the tokens) outputs that fill the
+// CUs take at least the slices the float cores cut them into: 50257 x 768 x
+// 8192 in 2730 (error against 64 bits 7.8e-7, in float 9.1e-7), x 2048 in
+// 1024 (5.0e-7, in one slice 6.9e-7; in float 5.9e-7).
+Plan choose_plan(int64_t M, int64_t N, int64_t K, int cus, bool wgrad) {
   int forced = -1;
   if (const char* e = getenv("TJH_SPLIT_TILE")) {
     for (int i = 0; i < kNumTiles; ++i) {
@@ -65,7 +70,11 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
   static const double uneven[kNumTiles] = {0.8, 0.8, 0.8, 0.3, 0.3, 0.3};
   static const double fixed[kNumTiles] = {9, 8, 7, 6, 5, 5};
   const int64_t blocks = cdiv(M, 128) * cdiv(N, 128);
-  const int64_t slice = blocks >= 2 * cus ? K + 1 : blocks >= cus ? 3200 : 400;
+  int64_t slice = blocks >= 2 * cus ? K + 1 : blocks >= cus ? 3200 : 400;
+  if (wgrad && blocks >= cus) {
+    slice = cdiv(K, 3) < 3200 ? cdiv(K, 3) : 3200;
+    if (slice < 1024) slice = 1024;
+  }
   int64_t smax = K / 64 < 64 ? K / 64 : 64;
   if (smax < 1) smax = 1;
   int64_t smin = cdiv(K, slice) < smax ? cdiv(K, slice) : smax;
@@ -119,7 +128,8 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
                               const float* residual, int64_t ldr, int act) {
   TJH_REQUIRE_INIT();
   TJH_ARG(M >= 0 && N >= 0 && K >= 0, "tjh_gemm_split: negative size");
-  TJH_ARG(bias_mode >= 0 && bias_mode <= 2, "tjh_gemm_split: bad bias_mode %d", bias_mode);
+  TJH_ARG(bias_mode >= 0 && bias_mode <= 3, "tjh_gemm_split: bad bias_mode %d", bias_mode);
+  TJH_ARG(bias_mode != 3 || act == 0, "tjh_gemm_split: bias_mode 3 takes no activation");
   TJH_ARG(bias_mode == 0 || bias, "tjh_gemm_split: bias_mode %d needs a bias pointer", bias_mode);
   TJH_ARG(act == 0 || act == 1 || act == 3, "tjh_gemm_split: bad activation %d", act);
   TJH_ARG(act != 3 || (residual && ldr >= N), "tjh_gemm_split: activation 3 needs residual (ld >= N)");
@@ -128,9 +138,9 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   TJH_ARG(lda >= (transA ? M : K) || (transA ? M : K) <= 1, "tjh_gemm_split: lda too small");
   TJH_ARG(ldb >= (transB ? K : N) || (transB ? K : N) <= 1, "tjh_gemm_split: ldb too small");
   TJH_ARG(ldc >= N, "tjh_gemm_split: ldc too small");
-  // A^T . B^T has no kernel here, and sums of fewer than two K steps nothing
-  // to gain: the float cores
-  if ((transA && transB) || K < 32) {
+  // A^T . B^T and row sums of an A stored [M][K] have no kernel here, and
+  // sums of fewer than two K steps nothing to gain: the float cores
+  if ((transA && transB) || (bias_mode == 3 && !transA) || K < 32) {
     if (act == 1) {  // which keep the pre-activation
       Scratch keep((size_t)(M * N) * sizeof(float));
       if (!keep.ok()) return set_error(TJH_ERR_OOM, "tjh_gemm_split: no scratch");
@@ -155,7 +165,7 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   // few rows: nothing to gain from the matrix cores
   if (!transA && transB && M <= kFewRows && g.vecA && g.vecB && cdiv(N, 4) < (int64_t(1) << 31))
     return gemm_rows(g, cus);
-  const Plan plan = choose_plan(M, N, K, cus);
+  const Plan plan = choose_plan(M, N, K, cus, transA);
   const TileCfg& tc = kTiles[plan.tile];
   g.tiles_m = (int)cdiv(M, tc.bm);
   g.tiles_n = (int)cdiv(N, tc.bn);
@@ -165,12 +175,15 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   int64_t splits = M * N < (int64_t(1) << 32) ? plan.splits : 1;
   g.kchunk = cdiv(cdiv(K, splits), BK) * BK;
   splits = cdiv(K, g.kchunk);
-  Scratch ws(splits > 1 ? (size_t)(splits * M * N) * sizeof(float) : 0);
+  // K slices: the products' partials, then the row sums'
+  const int64_t sums = bias_mode == 3 ? splits * M : 0;
+  Scratch ws(splits > 1 ? (size_t)(splits * M * N + sums) * sizeof(float) : 0);
   if (splits > 1 && !ws.ok()) {
     splits = 1;
     g.kchunk = cdiv(K, BK) * BK;
   }
   g.ws = splits > 1 ? ws.as<float>() : nullptr;
+  g.rsw = splits > 1 && sums ? g.ws + splits * M * N : nullptr;
   // tiles, K steps or loads that need a guard
   const bool edge = M % tc.bm || N % tc.bn || K % BK || !g.vecA || !g.vecB;
   launch_tile(plan.tile, g, dim3((unsigned)(g.tiles_m * g.tiles_n), (unsigned)splits), transA,

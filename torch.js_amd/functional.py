@@ -515,9 +515,9 @@ def linear(x, weight, bias=None):
         if rw and rb:
             # db = the row sums of g^T, accumulated by the dW GEMM itself
             db = empty((out_f,))
-            dw = _gemm(g2.T, x2, rowsum_out=db)
+            dw = _T._wgrad(g2, x2, db)
         elif rw:
-            dw = _gemm(g2.T, x2)
+            dw = _T._wgrad(g2, x2)
         elif rb:
             gc = g2 if g2.is_contiguous() else _k_contiguous(g2)
             db = _view_raw(_k_reduce("sum", gc, [0]), (out_f,))
@@ -566,9 +566,9 @@ def _linear_add(x, weight, bias, residual):
         dw = db = None
         if rw and rb:
             db = empty((out_f,))
-            dw = _gemm(g2.T, x2, rowsum_out=db)
+            dw = _T._wgrad(g2, x2, db)
         elif rw:
-            dw = _gemm(g2.T, x2)
+            dw = _T._wgrad(g2, x2)
         elif rb:
             gc = g2 if g2.is_contiguous() else _k_contiguous(g2)
             db = _view_raw(_k_reduce("sum", gc, [0]), (out_f,))
@@ -627,7 +627,7 @@ def _mlp_gelu(x, w1, b1, w2, b2, residual=None):
         if need[3] or need[4]:
             db2 = empty((d_out,)) if need[4] else None
             if need[3]:
-                dw2 = _gemm(g2.T, a, rowsum_out=db2)
+                dw2 = _T._wgrad(g2, a, db2)
             else:
                 db2 = _view_raw(_k_reduce("sum", g2, [0]), (d_out,))
         if need[0] or need[1] or need[2]:
@@ -637,7 +637,7 @@ def _mlp_gelu(x, w1, b1, w2, b2, residual=None):
                 dx = reshape_raw(_gemm(dh, w1d), lead + (d_in,))
             if need[1]:
                 db1 = empty((hid,)) if need[2] else None
-                dw1 = _gemm(dh.T, x2, rowsum_out=db1)
+                dw1 = _T._wgrad(dh, x2, db1)
             elif need[2]:
                 db1 = _view_raw(_k_reduce("sum", dh, [0]), (hid,))
         return [dx, dw1, db1, dw2, db2, g]
