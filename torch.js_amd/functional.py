@@ -494,11 +494,11 @@ def linear(x, weight, bias=None):
     x2 = reshape(x.detach(), (M, in_f))
     wd = weight.detach()
     bd = bias.detach().contiguous() if bias is not None else None
-    out2 = _gemm(x2, wd.T, bias=bd, bias_mode=1 if bd is not None else 0,
-                 recorded=_T._recorded(x, weight, bias))
-    out = reshape_raw(out2, lead + (out_f,))
     rx, rw = x.requires_grad, weight.requires_grad
     rb = bias is not None and bias.requires_grad
+    out2 = _gemm(x2, wd.T, bias=bd, bias_mode=1 if bd is not None else 0,
+                 recorded=_T._grad["enabled"] and (rx or rw or rb))
+    out = reshape_raw(out2, lead + (out_f,))
 
     def bwd(g):
         if isinstance(g, _T._CEGrad):
@@ -554,11 +554,11 @@ def _linear_add(x, weight, bias, residual):
     r2 = reshape(r if r.dtype == "float32" and r.is_contiguous() else r.float().contiguous(),
                  (M, out_f))
     out2 = empty((M, out_f))
-    _gemm(x2, wd.T, out=out2, bias=bd, bias_mode=1 if bd is not None else 0, aux=r2, act=3,
-          recorded=_T._recorded(x, weight, bias, residual))
-    out = reshape_raw(out2, lead + (out_f,))
     rx, rw = x.requires_grad, weight.requires_grad
     rb = bias is not None and bias.requires_grad
+    _gemm(x2, wd.T, out=out2, bias=bd, bias_mode=1 if bd is not None else 0, aux=r2, act=3,
+          recorded=_T._grad["enabled"] and (rx or rw or rb or residual.requires_grad))
+    out = reshape_raw(out2, lead + (out_f,))
 
     def bwd(g):
         g2 = reshape_raw(g, (M, out_f))

@@ -2764,7 +2764,11 @@ def _mat_operand(t):
 
 def _recorded(*ts):
     """Whether an op on these tensors records a graph node."""
-    return _grad["enabled"] and any(t is not None and t.requires_grad for t in ts)
+    if _grad["enabled"]:
+        for t in ts:
+            if t is not None and t.requires_grad:
+                return True
+    return False
 
 
 def _gemm(a, b, out=None, alpha=1.0, beta=0.0, bias=None, bias_mode=0, rowsum_out=None,
@@ -2848,8 +2852,8 @@ def _wgrad(g, x, rowsum_out=None):
     (2-norm) and 2.4e-4 in single ones (of their root mean square).  Smaller
     weights would gain as much (3072 x 768: 209 and 334 us), but theirs
     become 9e-6 and 1.6e-3: the float cores."""
-    large = -(-g.shape[1] // 128) * -(-x.shape[1] // 128) >= 256
-    return _gemm(g.T, x, rowsum_out=rowsum_out, recorded=not large)
+    small = ((g._shape[1] + 127) // 128) * ((x._shape[1] + 127) // 128) < 256
+    return _gemm(g.T, x, rowsum_out=rowsum_out, recorded=small)
 
 
 def _bgemm(a, b):
