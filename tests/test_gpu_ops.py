@@ -1067,6 +1067,29 @@ def test_attention_of_few_workgroups(torch, D, Tq, Tk, causal):
     assert np.linalg.norm(got - want) <= 1.5 * np.linalg.norm(rec - want) + 1e-7 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("D", [4, 16, 20, 40, 48, 52, 80, 84, 112, 116])
+@pytest.mark.parametrize("T,causal", [(64, False), (101, True)])
+def test_attention_head_dims_about_the_short_products(torch, D, T, causal):
+    """Forward and gradients at the head dims where the products over it
+    take fewer steps (up to 16, 48, 80, 112 of the padded dims) and beside."""
+    r = np.random.default_rng(D + T)
+    q, k, v, g = (f32(r.standard_normal((2, 2, T, D))) for _ in range(4))
+    t = [torch.tensor(a, requires_grad=True) for a in (q, k, v)]
+    y = torch.functional.scaled_dot_product_attention(*t, is_causal=causal)
+    y.backward(torch.tensor(g))
+    q, k, v, g = (a.astype(np.float64) for a in (q, k, v, g))
+    s = q @ k.swapaxes(-1, -2) / np.sqrt(D)
+    if causal:
+        s = np.where(np.tril(np.ones((T, T), bool)), s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    dp = g @ v.swapaxes(-1, -2)
+    ds = p * (dp - (p * dp).sum(-1, keepdims=True)) / np.sqrt(D)
+    for got, want in zip([y.detach()] + [a.grad for a in t],
+                         [p @ v, ds @ k, ds.swapaxes(-1, -2) @ q, p.swapaxes(-1, -2) @ g]):
+        check(got.numpy(), want, **RED)
+
+
 def test_attention_key_split_of_large_and_masked_scores(torch):
     """Scores of +-1e4 spread over the slices, and rows whose later slices
     underflow against the first."""

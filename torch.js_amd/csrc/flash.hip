@@ -10,9 +10,10 @@
 // never leave LDS / registers.
 //
 // Register layouts (one wave64 per 32 rows; lane l, l32 = l%32, h = l/32):
-//   * contraction over the head dim d uses, in MFMA step s (0..HD/2-1), the
-//     pair d = s (lanes h=0) and d = HD/2 + s (lanes h=1): each lane's HD/2
-//     operand values are one contiguous run of a row, read as 128-bit LDS
+//   * contraction over the head dim d uses, in MFMA step s (0..RUN-1, RUN =
+//     HD/2 or 8 less where the columns from 2 RUN on are empty), the pair d =
+//     s (lanes h=0) and d = RUN + s (lanes h=1): each lane's RUN operand
+//     values are one contiguous run of a row, read as 128-bit LDS
 //     loads;
 //   * a 32x32 accumulator register j of lane l holds C[8(j/4)+4h+j%4][l32],
 //     so contracting over that accumulator's row index in step s pairs the
@@ -186,13 +187,13 @@ __device__ __forceinline__ void store_tile(float* __restrict__ S, const floatx4 
   }
 }
 
-// The HD/2 operand values row[h*HD/2 ..] of an LDS tile row.
-template <int HD>
+// The RUN operand values row[h*RUN ..] of an LDS tile row.
+template <int HD, int RUN>
 __device__ __forceinline__ void lds_run(const float* __restrict__ S, int row, int h,
-                                        float (&x)[Hd<HD>::RUN]) {
-  const floatx4* p = reinterpret_cast<const floatx4*>(S + row * Hd<HD>::W + h * Hd<HD>::RUN);
+                                        float (&x)[RUN]) {
+  const floatx4* p = reinterpret_cast<const floatx4*>(S + row * Hd<HD>::W + h * RUN);
 #pragma unroll
-  for (int i = 0; i < Hd<HD>::RUN / 4; ++i) {
+  for (int i = 0; i < RUN / 4; ++i) {
     const floatx4 v = p[i];
     x[4 * i] = v.x;
     x[4 * i + 1] = v.y;
@@ -203,16 +204,16 @@ __device__ __forceinline__ void lds_run(const float* __restrict__ S, int row, in
 
 // The same run from global memory (rows >= T are zero; with GUARD, columns
 // >= D too), times `mul`.
-template <int HD, bool GUARD>
+template <int HD, bool GUARD, int RUN>
 __device__ __forceinline__ void gl_run(const float* __restrict__ base, int64_t st, int r, int T,
-                                       int D, int h, float mul, float (&x)[Hd<HD>::RUN]) {
+                                       int D, int h, float mul, float (&x)[RUN]) {
   if (r < T) {
     const floatx4* p =
-        reinterpret_cast<const floatx4*>(base + (int64_t)r * st + h * Hd<HD>::RUN);
+        reinterpret_cast<const floatx4*>(base + (int64_t)r * st + h * RUN);
 #pragma unroll
-    for (int i = 0; i < Hd<HD>::RUN / 4; ++i) {
+    for (int i = 0; i < RUN / 4; ++i) {
       floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (!GUARD || h * Hd<HD>::RUN + 4 * i < D) v = p[i];
+      if (!GUARD || h * RUN + 4 * i < D) v = p[i];
       x[4 * i] = v.x * mul;
       x[4 * i + 1] = v.y * mul;
       x[4 * i + 2] = v.z * mul;
@@ -220,7 +221,7 @@ __device__ __forceinline__ void gl_run(const float* __restrict__ base, int64_t s
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < Hd<HD>::RUN; ++i) x[i] = 0.f;
+    for (int i = 0; i < RUN; ++i) x[i] = 0.f;
   }
 }
 
@@ -235,24 +236,24 @@ __device__ __forceinline__ void lds_cols(const float* __restrict__ S, int l32, i
     for (int c = 0; c < Hd<HD>::NC; ++c) x[c][s] = S[kappa(s, h) * Hd<HD>::W + c * 32 + l32];
 }
 
-// acc = offset-step + sum over HD/2 steps of a[s] * b[s].  The offset step
+// acc = offset-step + sum over RUN steps of a[s] * b[s].  The offset step
 // adds off_a[m] * off_b[n] through the h = 0 lanes (a rank-1 update).
-template <int HD>
+template <int HD, int RUN>
 __device__ __forceinline__ floatx16 chain(float off_a, float off_b,
-                                          const float (&a)[Hd<HD>::RUN],
-                                          const float (&b)[Hd<HD>::RUN]) {
+                                          const float (&a)[RUN],
+                                          const float (&b)[RUN]) {
   floatx16 acc = mfma(off_a, off_b, zero16());
 #pragma unroll
-  for (int s = 0; s < Hd<HD>::RUN; ++s) acc = mfma(a[s], b[s], acc);
+  for (int s = 0; s < RUN; ++s) acc = mfma(a[s], b[s], acc);
   return acc;
 }
 
-template <int HD>
-__device__ __forceinline__ floatx16 chain0(const float (&a)[Hd<HD>::RUN],
-                                           const float (&b)[Hd<HD>::RUN]) {
+template <int HD, int RUN>
+__device__ __forceinline__ floatx16 chain0(const float (&a)[RUN],
+                                           const float (&b)[RUN]) {
   floatx16 acc = mfma(a[0], b[0], zero16());
 #pragma unroll
-  for (int s = 1; s < Hd<HD>::RUN; ++s) acc = mfma(a[s], b[s], acc);
+  for (int s = 1; s < RUN; ++s) acc = mfma(a[s], b[s], acc);
   return acc;
 }
 
@@ -293,7 +294,7 @@ __device__ __forceinline__ void zero_acc(floatx16 (&acc)[NC]) {
 // GUARD: Tk is not a multiple of 32 (the last key tile is partial), or D <
 // HD (padded columns).  PART: this workgroup takes one slice of the keys and
 // writes its running sums, which k_flash_merge adds up.
-template <int HD, bool GUARD, bool PART>
+template <int HD, bool GUARD, bool PART, int RUN>
 __global__ __launch_bounds__(256, occ_fwd<HD>()) void k_flash_fwd(FlashArgs a) {
   using S_ = Hd<HD>;
   __shared__ __attribute__((aligned(16))) float Ks[2][TILE * S_::W];
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(256, occ_fwd<HD>()) void k_flash_fwd(FlashArgs a) {
   const int kb0 = PART ? (int)blockIdx.y * a.kslice : 0;  // first key tile
   const int myq = q0 + l32;
 
-  float qf[S_::RUN];
+  float qf[RUN];
   gl_run<HD, GUARD>(Q, a.qs.t, myq, a.Tq, a.D, h, a.scale * kLog2e, qf);
   floatx16 acc[S_::NC];
   zero_acc(acc);
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(256, occ_fwd<HD>()) void k_flash_fwd(FlashArgs a) {
     const int k0 = kb * TILE;
     const bool skip = (a.causal && k0 > q0 + TILE - 1) || q0 >= a.Tq;
     if (!skip) {
-      float ka[S_::RUN];
+      float ka[RUN];
       lds_run<HD>(Ks[cur], l32, h, ka);
       floatx16 st = chain0<HD>(ka, qf);  // S^T[key][query], base-2 units
       float va[S_::NC][16];
@@ -810,7 +811,7 @@ __global__ __launch_bounds__(512, 1) void k_flash_dq_ds8(FlashArgs a) {
 // that wait never waits for the stores.  GUARD: Tq or Tk is not a multiple
 // of 32, or D < HD.
 constexpr int PROWS = 64;  // keys per workgroup
-template <int HD, bool GUARD, bool STORE>
+template <int HD, bool GUARD, bool STORE, int RUN>
 __global__ __launch_bounds__(256, occ_pair<HD>()) void k_flash_dkv_pair(FlashArgs a) {
   using S_ = Hd<HD>;
   __shared__ __attribute__((aligned(16))) float Qs[2][TILE * S_::W];
@@ -839,7 +840,7 @@ __global__ __launch_bounds__(256, occ_pair<HD>()) void k_flash_dkv_pair(FlashArg
   const int mykey = k0 + l32;
 
   // A: K rows (scaled to base-2 logits); B: V rows
-  float kv[S_::RUN];
+  float kv[RUN];
   if (role == 0)
     gl_run<HD, GUARD>(K, a.ks.t, mykey, a.Tk, a.D, h, a.scale * kLog2e, kv);
   else
@@ -847,7 +848,7 @@ __global__ __launch_bounds__(256, occ_pair<HD>()) void k_flash_dkv_pair(FlashArg
   // complete the loads here: a wait for them inside the loop would also
   // wait for every step's prefetch
 #pragma unroll
-  for (int i = 0; i < S_::RUN; ++i) asm volatile("" : "+v"(kv[i]));
+  for (int i = 0; i < RUN; ++i) asm volatile("" : "+v"(kv[i]));
   floatx16 acc[S_::NC];  // A: dV^T, B: dK^T
   zero_acc(acc);
   const float one = h == 0 ? 1.f : 0.f;
@@ -887,7 +888,7 @@ __global__ __launch_bounds__(256, occ_pair<HD>()) void k_flash_dkv_pair(FlashArg
     const bool edge = (a.causal && qq0 < k0 + TILE - 1) || (GUARD && qq0 + TILE > a.Tq);
     floatx16 x = zero16();  // A: P; B: dP - D, then dS
     if (!skip) {
-      float xa[S_::RUN];
+      float xa[RUN];
       // A: S[q][key] - lse[q] from Q rows; B: dP[q][key] - D[q] from dO rows
       lds_run<HD>(role == 0 ? Qs[cur] : Gs[cur], l32, h, xa);
       x = chain<HD>(off, one, xa, kv);
@@ -968,17 +969,27 @@ int cus_per_xcd() {
 
 int padded_hd(int64_t D) { return (int)((D + 31) / 32 * 32); }
 
+// Whether a head dim leaves 16 or more of the padded columns empty: the
+// products over it then take RUN = HD / 2 - 8 steps instead of HD / 2 (40 of
+// 48 at D = 80: 4 x 16 heads of 701 forward and backward 514 -> 490 us; 24 of
+// 32 at D = 40: 339 -> 315).
+template <int HD>
+bool short_run(const FlashArgs& a) { return a.D <= HD - 16; }
+
+template <int HD, bool PART>
+void launch_forward_part(const FlashArgs& a, dim3 grid) {
+  if (short_run<HD>(a))
+    tjh_launch(k_flash_fwd<HD, true, PART, HD / 2 - 8>, grid, dim3(256), 0, stream(), a);
+  else if ((a.Tk % TILE) || a.D != HD)
+    tjh_launch(k_flash_fwd<HD, true, PART, HD / 2>, grid, dim3(256), 0, stream(), a);
+  else
+    tjh_launch(k_flash_fwd<HD, false, PART, HD / 2>, grid, dim3(256), 0, stream(), a);
+}
+
 template <int HD>
 void launch_forward(const FlashArgs& a, unsigned grid) {
-  const bool guard = (a.Tk % TILE) || a.D != HD;
-  if (a.part && guard)
-    tjh_launch(k_flash_fwd<HD, true, true>, dim3(grid, a.nsl), dim3(256), 0, stream(), a);
-  else if (a.part)
-    tjh_launch(k_flash_fwd<HD, false, true>, dim3(grid, a.nsl), dim3(256), 0, stream(), a);
-  else if (guard)
-    tjh_launch(k_flash_fwd<HD, true, false>, dim3(grid), dim3(256), 0, stream(), a);
-  else
-    tjh_launch(k_flash_fwd<HD, false, false>, dim3(grid), dim3(256), 0, stream(), a);
+  if (a.part) launch_forward_part<HD, true>(a, dim3(grid, a.nsl));
+  else launch_forward_part<HD, false>(a, dim3(grid));
 }
 
 // Key tiles per slice of a forward pass of BH heads, or 0 where its blocks
@@ -1008,10 +1019,12 @@ int launch_backward(FlashArgs a, int64_t BH, const int64_t* dq_st, float* dq) {
   if (a.dsblk) {
     a.nblk = (int)cdiv(a.Tk, PROWS);
     const unsigned gk = (unsigned)(BH * a.nblk);
-    if (ragged)
-      tjh_launch(k_flash_dkv_pair<HD, true, true>, dim3(gk), dim3(256), 0, stream(), a);
+    if (short_run<HD>(a))
+      tjh_launch(k_flash_dkv_pair<HD, true, true, HD / 2 - 8>, dim3(gk), dim3(256), 0, stream(), a);
+    else if (ragged)
+      tjh_launch(k_flash_dkv_pair<HD, true, true, HD / 2>, dim3(gk), dim3(256), 0, stream(), a);
     else
-      tjh_launch(k_flash_dkv_pair<HD, false, true>, dim3(gk), dim3(256), 0, stream(), a);
+      tjh_launch(k_flash_dkv_pair<HD, false, true, HD / 2>, dim3(gk), dim3(256), 0, stream(), a);
   } else {
     a.nblk = (int)cdiv(a.Tk, ROWS);
     const unsigned gk = (unsigned)(BH * a.nblk);
