@@ -982,6 +982,55 @@ def test_gemm_split_not_finite_every_tile(torch, monkeypatch, tile, ta, tb):
     assert np.array_equal(got[257][fin], want32[257][fin])
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0)])
+def test_gemm_split_not_finite_in_slices_of_k(torch, ta, tb):
+    """The same where K is cut into slices, beside finite blocks, which keep
+    their sums: rows 32 to 63 of C are one block of rows."""
+    r = np.random.default_rng(3 + ta)
+    M, N, K = 100, 70, 6001
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    A[40, 6000], A[41, 17], A[41, 5000] = np.inf, np.inf, -np.inf
+    got = _raw_split(torch, ta, tb, np.ascontiguousarray(A.T) if ta else A,
+                     np.ascontiguousarray(B.T) if tb else B, M, N, K)
+    assert np.array_equal(got[40], np.where(B[6000] > 0, np.inf, -np.inf))
+    assert (np.isnan(got[41]) | np.isinf(got[41])).all()  # inf - inf where the signs agree
+    assert np.array_equal(np.isnan(got[41]), np.sign(B[17]) == np.sign(B[5000]))
+    ok = [i for i in range(M) if i not in (40, 41)]
+    want = A[ok].astype(np.float64) @ B.astype(np.float64)
+    check_floor(got[ok], want, A[ok] @ B)
+
+
+def test_gemm_split_not_finite_costs_a_float_product(torch):
+    """A NaN in every row of A: every block of the product is formed again on
+    the float matrix cores.  These take about twice the split products' time
+    and read their operands unstaged, so ten times the clean product's time
+    is far above it (and an order of magnitude below what one multiply-add
+    after the other takes)."""
+    import time
+    from torchjs_amd import _lib as L
+    M, N, K = 2048, 3072, 768
+    r = np.random.default_rng(1)
+    an = f32(r.standard_normal((M, K)))
+    bad = an.copy()
+    bad[:, 5] = np.nan
+    b, c = torch.tensor(f32(r.standard_normal((N, K)))), torch.zeros(M, N)
+
+    def best(a):
+        t = []
+        for _ in range(6):
+            torch.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(5):
+                L.check(L.lib().tjh_gemm_split(0, 1, M, N, K, 1.0, a.data_ptr(), K, b.data_ptr(), K, 0.0,
+                                               c.data_ptr(), N, None, 0, None, 0, 0))
+            torch.synchronize()
+            t.append(time.perf_counter() - t0)
+        return min(t)
+    clean = best(torch.tensor(an))
+    assert best(torch.tensor(bad)) <= 10 * clean
+    assert np.isnan(c.numpy()).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 512, 768), (200, 300, 1000), (64, 64, 8192)])
 def test_gemm_split_error_of_float_products(torch, M, N, K):
     """Against 64 bits the three-part products are no further off than a

@@ -245,6 +245,45 @@ constexpr int gemm_waves_per_simd(int wm, int wn) { return wm * wn >= 64 * 96 ? 
 //   that a sum meets both directions.
 constexpr int kFlip = 32;
 
+// The 32 x 32 block of products over [kbeg, kend) that holds row `row` (of
+// this lane's A value) and column `col` (of its B value; both clamped to the
+// product) on the float matrix cores, in the accumulator layout above.  Lane
+// half h takes k = 8 h .. + 7 of each 16, so a lane's values of an operand
+// with k contiguous are two 128-bit loads.
+template <bool TA, bool TB>
+__device__ __forceinline__ floatx16 float_block(const GemmArgs& g, int64_t row, int64_t col, int h,
+                                                int64_t kbeg, int64_t kend) {
+  if (row >= g.M) row = g.M - 1;
+  if (col >= g.N) col = g.N - 1;
+  const float* __restrict__ a = TA ? g.A + row : g.A + row * g.lda;
+  const float* __restrict__ b = TB ? g.B + col * g.ldb : g.B + col;
+  floatx16 s;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll 1
+  for (int64_t k0 = kbeg; k0 < kend; k0 += 16) {
+    const int64_t k = k0 + 8 * h;
+    float x[8], y[8];
+    if (k0 + 16 <= kend) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        x[q] = TA ? a[(k + q) * g.lda] : a[k + q];
+        y[q] = TB ? b[k + q] : b[(k + q) * g.ldb];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        x[q] = k + q < kend ? (TA ? a[(k + q) * g.lda] : a[k + q]) : 0.f;
+        y[q] = k + q < kend ? (TB ? b[k + q] : b[(k + q) * g.ldb]) : 0.f;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(x[q], y[q], s, 0, 0, 0);
+  }
+  return s;
+}
+
 template <int BM, int BN, int WR, int WC, bool TA, bool TB, bool EDGE>
 __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)) void k_gemm_split(
     GemmArgs g) {
@@ -450,41 +489,34 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
     else if (g.bias_mode == 2) v += g.bias[row];
     *cp = epilogue_act(g, row, col, v);
   };
-  // An infinity or NaN among the operands (or a finite value that rounds to
-  // infinity in bfloat16) makes parts of the split NaN: a wave whose sums
-  // are not all finite forms them again from the floats themselves, with
-  // the infinities and NaNs of float arithmetic.  0 * x is 0 for finite x
-  // and NaN otherwise.
-  {
-    float z[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) z[r & 3] = __builtin_fmaf(acc[i][j][r], 0.f, z[r & 3]);
-    const float zz = (z[0] + z[1]) + (z[2] + z[3]);
-    if (__any(!(zz == 0.f))) {
-#pragma unroll 1
-      for (int e = 0; e < FM * FN * 16; ++e) {
-        const int r = e & 15, ij = e >> 4;
-        const int64_t row = r0 + (ij / FN) * 32 + 8 * (r >> 2) + (r & 3), col = c0 + (ij % FN) * 32;
-        if (EDGE && (row >= g.M || col >= g.N)) continue;
-        float s = 0.f;
-#pragma unroll 1
-        for (int64_t k = kbeg; k < kend; ++k) {
-          const float a = TA ? A[k * g.lda + row] : A[row * g.lda + k];
-          s = __builtin_fmaf(a, TB ? B[col * g.ldb + k] : B[k * g.ldb + col], s);
-        }
-        finish(row, col, s);
-      }
-      return;
-    }
-  }
   // the sign of this lane's column after the last K tile; odd rows carry the
   // other one
   const int64_t kt = kend > kbeg ? cdiv(kend - kbeg, BK) : 1;
   const float sign = (l32 + (kt - 1) / kFlip) & 1 ? -1.f : 1.f, alpha = g.alpha * sign;
+  // An infinity or NaN among the operands (or a finite value that rounds to
+  // infinity in bfloat16) makes parts of the split NaN: the 32 x 32 blocks
+  // whose sums are not all finite are formed again from the floats
+  // themselves, on the float matrix cores, with the infinities and NaNs of
+  // float arithmetic.  0 * x is 0 for finite x and NaN otherwise.  2048 x
+  // 3072 x 768 takes 75 us, with a NaN in every row 243 us (11.3 ms by
+  // multiply-adds one after the other, 89 us on gemm.hip's tiles).
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      float z0 = 0.f, z1 = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        z0 = __builtin_fmaf(acc[i][j][r], 0.f, z0);
+        z1 = __builtin_fmaf(acc[i][j][r + 1], 0.f, z1);
+      }
+      if (__any(!(z0 + z1 == 0.f))) {
+        acc[i][j] = float_block<TA, TB>(g, m0 + wm * WM + i * 32 + l32, n0 + wn * WN + j * 32 + l32,
+                                        h, kbeg, kend);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] *= r & 1 ? -sign : sign;
+      }
+    }
   auto each = [&](auto&& put) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
