@@ -1000,6 +1000,27 @@ def test_gemm_split_not_finite_in_slices_of_k(torch, ta, tb):
     check_floor(got[ok], want, A[ok] @ B)
 
 
+@pytest.mark.parametrize("tile", SPLIT_TILES)
+@pytest.mark.parametrize("ta,tb,K", [(0, 1, 70), (1, 0, 96), (0, 0, 6000)])
+def test_gemm_split_zeros_are_positive_every_tile(torch, monkeypatch, tile, ta, tb, K):
+    """Sums that are exactly zero, of zeros of both signs or of terms that
+    cancel, are +0, in slices of K too."""
+    monkeypatch.setenv("TJH_SPLIT_TILE", tile)
+    r = np.random.default_rng(K)
+    M, N = 260, 100
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    A[:128] = 0
+    A[64:128] *= -1
+    A[128:192] = 0
+    A[128:192, 3], A[128:192, K - 1] = 1, -1
+    B[K - 1] = B[3]
+    B[:, 60:] = 0
+    got = _raw_split(torch, ta, tb, np.ascontiguousarray(A.T) if ta else A,
+                     np.ascontiguousarray(B.T) if tb else B, M, N, K)
+    assert (got[:192] == 0).all() and (got[:, 60:] == 0).all()
+    assert not np.signbit(got[got == 0]).any()
+
+
 def test_gemm_split_not_finite_costs_a_float_product(torch):
     """A NaN in every row of A: every block of the product is formed again on
     the float matrix cores.  These take about twice the split products' time

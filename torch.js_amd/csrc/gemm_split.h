@@ -490,9 +490,10 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
     *cp = epilogue_act(g, row, col, v);
   };
   // the sign of this lane's column after the last K tile; odd rows carry the
-  // other one
+  // other one.  It is taken back by a multiply-add with +0, which a sum that
+  // is exactly zero leaves as +0, as the float cores do.
   const int64_t kt = kend > kbeg ? cdiv(kend - kbeg, BK) : 1;
-  const float sign = (l32 + (kt - 1) / kFlip) & 1 ? -1.f : 1.f, alpha = g.alpha * sign;
+  const float sign = (l32 + (kt - 1) / kFlip) & 1 ? -1.f : 1.f, alpha = g.alpha;
   // An infinity or NaN among the operands (or a finite value that rounds to
   // infinity in bfloat16) makes parts of the split NaN: the 32 x 32 blocks
   // whose sums are not all finite are formed again from the floats
@@ -526,7 +527,8 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int ro = i * 32 + 8 * (r >> 2) + (r & 3);
-          if (!EDGE || r0 + ro < g.M) put(r & 1 ? -acc[i][j][r] : acc[i][j][r], ro, j * 32);
+          if (!EDGE || r0 + ro < g.M)
+            put(__builtin_fmaf(acc[i][j][r], r & 1 ? -sign : sign, 0.f), ro, j * 32);
         }
       }
   };
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
     // raw partial sums; the reduce kernel applies alpha / beta / bias
     float* __restrict__ W = Wp + r0 * g.N + c0;
     const int64_t ld = g.N;
-    each([&](float a, int ro, int co) { W[ro * ld + co] = sign * a; });
+    each([&](float a, int ro, int co) { W[ro * ld + co] = a; });
     return;
   }
   float* __restrict__ Cb = C + r0 * g.ldc + c0;
@@ -564,7 +566,7 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
     else if (act == 1) run(IConst<1>());
     else run(IConst<3>());
   } else {
-    each([&](float a, int ro, int co) { finish(r0 + ro, c0 + co, sign * a); });
+    each([&](float a, int ro, int co) { finish(r0 + ro, c0 + co, a); });
   }
 }
 
