@@ -14,27 +14,37 @@
 // Products.  v_mfma_f32_32x32x2_f32 does 64 FLOP per cycle and SIMD, the
 // bf16 32x32x16 form 1024.  Each float is split into three bf16 parts that
 // sum to it exactly (split2 below) and six of the nine part products are
-// added up in float: 2.67 times the float rate, with an error against 64
-// bits under the float form's (a 768-term product of normal values: 4.2e-7
-// against 5.0e-7 rel.; 8192 terms: 1.45e-6 against 1.7e-6), because a
-// 16-term step meets fewer roundings.  8192 x 3072 x 768 takes 317-350 us on
-// the float cores and 193-240 us here, 8192 x 768 x 50257 4.7 and 3.4 ms,
-// 777 x 2304 x 768 50 and 30 us.  What bounds the large ones is power: with
-// random operands the clock falls to 1.9 GHz (an all-zero product runs at
-// 2.36 GHz and 309 TFLOP/s, a random one of 8192^3 at 214-238), so data
-// moved per product counts as much as issue slots.
+// added up in float, 2.67 times the float rate.
+//
+// Sums.  A running sum in the matrix cores is rounded at every instruction:
+// at every second k in the float form, six times in 16 k's here.  So there
+// are two running sums, one of the product of the leading parts, and one of
+// the five others, 2^-7 and less of it, whose roundings do not count: one
+// rounding in 16 k's.  Against 64 bits, single slices, normal values: 768
+// terms 1.6e-7 (float 5.0e-7, one sum of all six 4.2e-7), 4096 terms 4.0e-7
+// (float 1.1e-6); products of positive values or of a constant and values in
+// [0, 1) alike (768 terms 1.2e-7 and 1.4e-7, float 3.5e-7 and 3.7e-7, one sum
+// 4.0e-7 and 6.2e-7).  The instruction also loses the low bits of its small
+// terms to one side, downwards: the mean error of 8192 x 3072 x 768 is 6
+// standard errors from zero.  Every second row of A and column of B is
+// negated, so that neighbouring elements lose to opposite sides (under 1).
+//
+// 8192 x 3072 x 768 takes 317-350 us on the float cores and 209-228 us here,
+// 50257 x 768 x 8192 (A^T B) 4.8 and 3.6 ms, 777 x 2304 x 768 50 and 34 us.
+// What bounds the large ones is power: with random operands the clock falls
+// to 1.9 GHz, so data moved per product counts as much as issue slots.
 //
 // Tiling (a workgroup of WR x WC waves): block tile BM x BN, K step 16; each
-// wave owns a (BM / WR) x (BN / WC) sub-tile of 32x32 MFMA blocks.  Operand
-// tiles are loaded as floats into registers one step ahead (two steps on
-// wave tiles of 64 x 64 or less, which have the registers: 250 -> 214 us for
-// 8192 x 3072 x 768 on 128 x 128), split there once per workgroup, and
-// stored as three planes of bf16 in one of two LDS buffers.  The larger wave
-// tiles read and split less per product but leave CUs idle on small outputs:
-//   256 x 256, 8 waves of 128 x 64, one workgroup per CU
-//   256 x 192, 8 waves of 64 x 96, one per CU
-//   256 x 128, 4 waves of 128 x 64, two per CU
-//   128 x 128 / 128 x 64 / 64 x 64, 4 waves, three or more per CU
+// wave owns a (BM / WR) x (BN / WC) sub-tile of 32x32 MFMA blocks, at most 64
+// x 64, whose two sums take 128 registers.  Operand tiles are loaded as floats
+// into registers one step ahead (two steps on the smaller wave tiles; on 64 x
+// 64 the second set is no gain: 8192 x 3072 x 768 226 us with, 213 without),
+// split there once per workgroup, and stored as three planes of bf16 in one
+// of two LDS buffers.
+//   256 x 128, 8 waves of 64 x 64, one workgroup per CU
+//   128 x 128, 4 waves of 64 x 64, two per CU
+//   128 x 64, 4 waves of 64 x 32, three per CU
+//   64 x 64, 4 waves of 32 x 32, four per CU
 // Small outputs with long K are split over K; partials are summed by a
 // second pass in a fixed order (deterministic).
 // MFMA operand layout (32x32x16 bf16): lane l feeds A[m = l%32][k = 8*(l/32)
@@ -63,9 +73,10 @@ namespace tjh {
 // bfloat16 of what is left.  Three times eight significant bits hold the 24
 // of a float: the sum is exact while the parts stay above the smallest
 // bfloat16 (2^-133), so for |x| >= 2^-109; below, an absolute error of at
-// most 2^-134 remains.  |m| <= 2^-9 |x| and |l| <= 2^-18 |x|, so of the
-// nine products of two split numbers the three not formed (m l, l m, l l)
-// are under 2^-26 of the product, a quarter of one float rounding.
+// most 2^-134 remains.  For 1 <= |x| < 2, |m| <= 2^-8 and |l| <= 2^-17, so
+// of the nine products of two split numbers the three not formed (m l, l m,
+// l l) are at most 2^-24 + 2^-34 of the product, one float rounding of it
+// (a tenth of that in the root mean square over normal values).
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -193,7 +204,7 @@ struct Tile {
   }
   // Splits the tile and stores its parts in LDS, `part` bytes apart, outer
   // index o negated where o + flip is odd (kFlip below).
-  __device__ __forceinline__ void store(char* __restrict__ S, int part, int flip) const {
+  __device__ __forceinline__ void store(char* __restrict__ S, int part) const {
 #pragma unroll
     for (int i = 0; i < I; ++i) {
       if (!has(i)) continue;
@@ -201,7 +212,7 @@ struct Tile {
       at(i, o, kq);
 #pragma unroll
       for (int w = 0; w < W; ++w) {
-        const float sign = (o + w + flip) & 1 ? -1.f : 1.f;
+        const float sign = (o + w) & 1 ? -1.f : 1.f;
         uintx4 h, m, l;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -234,16 +245,9 @@ __device__ __forceinline__ int xcd_tile(int bid, int n) {
 
 // Wave tiles that keep 96 accumulator registers or more run two waves per
 // SIMD (256 registers each), smaller ones three or more.
-constexpr int gemm_waves_per_simd(int wm, int wn) { return wm * wn >= 64 * 96 ? 2 : wm * wn >= 64 * 64 ? 3 : 4; }
-
-// The bf16 matrix cores round their sums down (toward minus infinity), not
-// to the nearest, so a long sum drifts and so does the mean of a product (43
-// standard errors for 8192 x 3072 x 768).  Two changes of sign undo it:
-//   every second row of A and column of B is negated, so that the sums of
-//   neighbouring elements round in opposite directions;
-//   every kFlip K tiles the running sums and the signs of A are negated, so
-//   that a sum meets both directions.
-constexpr int kFlip = 32;
+constexpr int gemm_waves_per_simd(int wm, int wn) {
+  return wm * wn >= 64 * 64 ? 2 : wm * wn >= 64 * 32 ? 3 : 4;
+}
 
 // The 32 x 32 block of products over [kbeg, kend) that holds row `row` (of
 // this lane's A value) and column `col` (of its B value; both clamped to the
@@ -324,13 +328,16 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   const int wm = wid / WC, wn = wid % WC;
   const int l32 = lane & 31, h = lane >> 5;
 
-  floatx16 acc[FM][FN];
+  floatx16 acc[FM][FN], low[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        acc[i][j][r] = 0.f;
+        low[i][j][r] = 0.f;
+      }
 
   // A: logical [M][K]; stored [M][K] (!TA) or [K][M] (TA)
   // B: logical [K][N]; as an "outer = n" tile it is stored [N][K] when TB
@@ -355,18 +362,11 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   auto stage = [&](int64_t t, TileA& xa, TileB& xb) {
     char* S = lds + (t & 1) * BUF;
     if (TA && row_sums) xa.sum(rsum);
-    xa.store(S, PA, (int)(t / kFlip) & 1);
-    xb.store(S + 3 * PA, PB, 0);
+    xa.store(S, PA);
+    xb.store(S + 3 * PA, PB);
   };
-  // The six products of a K tile, the smallest terms first: the rounding of
-  // the running sum is the only float rounding they meet.
+  // the six products of a K tile, the smallest terms first
   auto compute = [&](int64_t t) {
-    if (t % kFlip == 0 && t > 0) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = -acc[i][j];
-    }
     const char* S = lds + (t & 1) * BUF;
     const int at = (h << 9) + ((l32 ^ (h << 2)) << 4);
     const char* as = S + wm * FM * kBlk + at;
@@ -387,9 +387,10 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
 #pragma unroll
       for (int u = 0; u < 6; ++u)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[PI[u]], bf[j][PJ[u]], acc[i][j],
-                                                              0, 0, 0);
+        for (int j = 0; j < FN; ++j) {
+          floatx16& to = u < 5 ? low[i][j] : acc[i][j];
+          to = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[PI[u]], bf[j][PJ[u]], to, 0, 0, 0);
+        }
     }
   };
 
@@ -489,11 +490,14 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
     else if (g.bias_mode == 2) v += g.bias[row];
     *cp = epilogue_act(g, row, col, v);
   };
-  // the sign of this lane's column after the last K tile; odd rows carry the
-  // other one.  It is taken back by a multiply-add with +0, which a sum that
-  // is exactly zero leaves as +0, as the float cores do.
-  const int64_t kt = kend > kbeg ? cdiv(kend - kbeg, BK) : 1;
-  const float sign = (l32 + (kt - 1) / kFlip) & 1 ? -1.f : 1.f, alpha = g.alpha;
+  // The sign of this lane's column; odd rows carry the other one.  It is
+  // taken back by a multiply-add with +0, which a sum that is exactly zero
+  // leaves as +0, as the float cores do.
+  const float sign = l32 & 1 ? -1.f : 1.f, alpha = g.alpha;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] += low[i][j];
   // An infinity or NaN among the operands (or a finite value that rounds to
   // infinity in bfloat16) makes parts of the split NaN: the 32 x 32 blocks
   // whose sums are not all finite are formed again from the floats
@@ -573,8 +577,7 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
 struct TileCfg {
   int bm, bn, wr, wc;  // block tile, wave rows and columns
 };
-constexpr TileCfg kTiles[] = {{256, 256, 2, 4}, {256, 192, 4, 2}, {256, 128, 2, 2},
-                              {128, 128, 2, 2}, {128, 64, 2, 2},  {64, 64, 2, 2}};
+constexpr TileCfg kTiles[] = {{256, 128, 4, 2}, {128, 128, 2, 2}, {128, 64, 2, 2}, {64, 64, 2, 2}};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 template <int BM, int BN, int WR, int WC, bool EDGE>
@@ -601,7 +604,7 @@ void launch_split(const GemmArgs& g, dim3 grid, int ta, int tb, bool edge) {
 
 /* tjh_gemm (batch 1) for a result that no gradient is taken through: float
  * products formed from three bf16 parts of each operand.  Its error against
- * 64 bits is under tjh_gemm's, but its roundings are others.  (Elements under
+ * 64 bits is no larger than tjh_gemm's, but its roundings are others.  (Elements under
  * 2^-109 in magnitude keep an absolute error of up to 2^-134.)
  * act 0: nothing; 1: C = GELU(v); 3: C = residual + v, with residual [M][N]
  * at row stride ldr, not overlapping C.  bias_mode 0 to 3 as tjh_gemm, 3

@@ -14,8 +14,6 @@ extern template void launch_split<0>(const GemmArgs&, dim3, int, int, bool);
 extern template void launch_split<1>(const GemmArgs&, dim3, int, int, bool);
 extern template void launch_split<2>(const GemmArgs&, dim3, int, int, bool);
 extern template void launch_split<3>(const GemmArgs&, dim3, int, int, bool);
-extern template void launch_split<4>(const GemmArgs&, dim3, int, int, bool);
-extern template void launch_split<5>(const GemmArgs&, dim3, int, int, bool);
 
 namespace {
 
@@ -27,76 +25,75 @@ struct Plan {
 // Picks the tile and the K slices of least estimated time, the sum of, in
 // microseconds:
 //   the larger of (a) the products at the tile's full rate, stretched by
-//   how unevenly the workgroups fill the CUs and (b) one workgroup's K steps
+//   how unevenly the workgroups fill the CUs, and (b) one workgroup's K steps
 //   at the pace of a workgroup alone on its CU, which is fetch latency for
 //   the small tiles;
 //   a fixed cost (first fetch, epilogue);
-//   with slices, writing and adding the partials (5 TB/s) in one launch more.
-// Rates are TFLOP/s with the CUs full, as measured on GPT-2's products
-// (8192 tokens, 768 to 50257 wide; the chip's power limit holds the clock
-// near 1.9 GHz there, where the six bf16 products allow 320): the larger
-// the wave tile the fewer LDS bytes and operand splits per product.  The
-// steps alone are from products of 8192 x 768 x 768 (96 to 192 of the large
-// tiles) and 777 x 768 x 768 (42 to 156 of the small ones).  A CU that runs
-// two or three small workgroups hides most of an uneven last round (8192 x
-// 2304 x 768 in 4.5 tiles of 128 x 128 per CU: 157 us, 152 at the full
-// rate), one or two large ones hide little (256 x 128, 2.25 per CU: 184).
+//   with slices, writing and adding the partials in one launch more.
+// The constants are a least-squares fit to 2433 times of 111 products (12 to
+// 8192 rows, 10 to 50257 columns, 40 to 9000 terms, every tile, 1 to 48
+// slices), 8% root mean square; its choices are 3.5% off the fastest on
+// average.  Rates are TFLOP/s with the CUs full (the chip's power limit holds
+// the clock near 1.9 GHz there, where the six bf16 products allow 320).  A
+// first round in which every CU holds at least one workgroup, but not its
+// fill of `cap`, loses `part` of the idle share, later rounds `uneven`.
+// With A transposed the widest tile, which reads the tall operand least, is
+// 4% faster than the others (50257 x 768 x 8192: 3.59 ms, 3.79 in 128 x 128).
 //
-// The rounding of a sum grows with the terms of its slice, and the float
-// cores split what cannot fill the CUs into slices of 256 k's and more: here
-// slices are kept to 400 where the output has fewer 128 x 128 tiles than
-// there are CUs, and to 3200 where it has fewer than twice as many, which
-// keeps the error at the float products' (logits of GPT-2 over 777 tokens,
-// 64-bit reference: 8.2e-7 off in single slices, 7.1e-7 so, 7.1e-7 in float).
+// The rounding of a sum grows with the root of its slice's terms.  The float
+// cores cut what cannot fill half the CUs with 128 x 128 tiles into slices of
+// 64 k's and more, and what cannot fill them twice into 256 and more.  The two
+// sums here round an eighth as often, so slices of eight times that length
+// err no more: 512 and 2048 (777 x 768 x 768: 1.1e-7 off 64 bits in two
+// slices, 1.6e-7 in one, 1.6e-7 in float; 777 x 1536 x 384 in one: 1.1e-7,
+// in float 1.5e-7).
 //
-// TJH_SPLIT_TILE=BMxBN forces a tile (read on every call, so a test can
-// sweep the tiles in one process).
-//
-// With A transposed (a weight gradient, K the tokens) outputs that fill the
-// CUs take at least the slices the float cores cut them into: 50257 x 768 x
-// 8192 in 2730 (error against 64 bits 7.8e-7, in float 9.1e-7), x 2048 in
-// 1024 (5.0e-7, in one slice 6.9e-7; in float 5.9e-7).
-Plan choose_plan(int64_t M, int64_t N, int64_t K, int cus, bool wgrad) {
+// TJH_SPLIT_TILE=BMxBN forces a tile and BMxBN:S its slices (read on every
+// call, so a test can sweep them in one process).
+Plan choose_plan(int64_t M, int64_t N, int64_t K, int cus, bool ta) {
   int forced = -1;
+  int64_t slices = 0;
   if (const char* e = getenv("TJH_SPLIT_TILE")) {
     for (int i = 0; i < kNumTiles; ++i) {
       char buf[32];
       snprintf(buf, sizeof(buf), "%dx%d", kTiles[i].bm, kTiles[i].bn);
-      if (strncmp(buf, e, strlen(buf)) == 0) forced = i;
+      const size_t n = strlen(buf);
+      if (strncmp(buf, e, n) == 0 && (e[n] == 0 || e[n] == ':')) {
+        forced = i;
+        if (e[n] == ':') slices = atoi(e + n + 1);
+      }
     }
   }
-  static const double rate[kNumTiles] = {212, 200, 203, 190, 160, 125};
-  static const double step[kNumTiles] = {1.84, 1.5, 1.2, 0.62, 0.55, 0.5};
-  static const double uneven[kNumTiles] = {0.8, 0.8, 0.8, 0.3, 0.3, 0.3};
-  static const double fixed[kNumTiles] = {9, 8, 7, 6, 5, 5};
+  static const double rate[kNumTiles] = {201, 200, 155, 120};
+  static const double step[kNumTiles] = {1.11, 0.82, 0.61, 0.51};
+  static const double fixed[kNumTiles] = {8, 7.8, 6.8, 6.7};
+  static const double part[kNumTiles] = {1.2, 0.64, 0.97, 1.2};
+  static const double uneven[kNumTiles] = {0.75, 0.59, 0.29, 0.41};
+  static const int cap[kNumTiles] = {1, 2, 3, 4};
   const int64_t blocks = cdiv(M, 128) * cdiv(N, 128);
-  int64_t slice = blocks >= 2 * cus ? K + 1 : blocks >= cus ? 3200 : 400;
-  if (wgrad && blocks >= cus) {
-    slice = cdiv(K, 3) < 3200 ? cdiv(K, 3) : 3200;
-    if (slice < 1024) slice = 1024;
-  }
+  const int64_t slice = 2 * blocks < cus ? 512 : blocks < 2 * cus ? 2048 : K + 1;
   int64_t smax = K / 64 < 64 ? K / 64 : 64;
   if (smax < 1) smax = 1;
-  int64_t smin = cdiv(K, slice) < smax ? cdiv(K, slice) : smax;
-  if (smin < 1) smin = 1;
+  const int64_t smin = cdiv(K, slice) < smax ? cdiv(K, slice) : smax;
   Plan best{kNumTiles - 1, 1};
   double best_t = 1e300;
   for (int i = 0; i < kNumTiles; ++i) {
     if (forced >= 0 && i != forced) continue;
     const TileCfg& t = kTiles[i];
     const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
-    const double work = 2e-6 * tiles * t.bm * t.bn * K / rate[i];
+    const double work = 2e-6 * tiles * t.bm * t.bn * K / (ta && i == 0 ? 1.04 * rate[i] : rate[i]);
     // slices that make whole rounds of the CUs
     for (int64_t rounds = 0; rounds <= 6; ++rounds) {
       int64_t s = rounds * cus / tiles;
       s = s < smin ? smin : s > smax ? smax : s;
-      const double n = (double)tiles * s / cus;
-      const double most = (double)cdiv(tiles * s, cus);
-      const double full = work * (n < 1 ? 1 : 1 + uneven[i] * (most / n - 1));
+      if (slices > 0) s = slices;
+      const double n = (double)tiles * s / cus;  // workgroups a CU
+      const double idle = n <= cap[i] ? part[i] * (cdiv(tiles * s, cus) / n - 1)
+                                      : uneven[i] * (cdiv(tiles * s, cap[i] * cus) * cap[i] / n - 1);
+      const double full = n < 1 ? work : work * (1 + idle);
       const double alone = cdiv(cdiv(K, s), BK) * step[i];
-      double us = full > alone ? full : alone;
-      us += fixed[i];
-      if (s > 1) us += 5 + 8e-6 * s * M * N / 5;
+      double us = (full > alone ? full : alone) + fixed[i];
+      if (s > 1) us += 1.8 + 8e-6 * s * M * N / 5.6;
       if (us < best_t) {
         best_t = us;
         best = Plan{i, s};
@@ -111,9 +108,7 @@ void launch_tile(int ti, const GemmArgs& g, dim3 grid, int ta, int tb, bool edge
     case 0: launch_split<0>(g, grid, ta, tb, edge); break;
     case 1: launch_split<1>(g, grid, ta, tb, edge); break;
     case 2: launch_split<2>(g, grid, ta, tb, edge); break;
-    case 3: launch_split<3>(g, grid, ta, tb, edge); break;
-    case 4: launch_split<4>(g, grid, ta, tb, edge); break;
-    default: launch_split<5>(g, grid, ta, tb, edge); break;
+    default: launch_split<3>(g, grid, ta, tb, edge); break;
   }
 }
 

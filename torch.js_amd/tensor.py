@@ -2846,7 +2846,7 @@ def _wgrad(g, x, rowsum_out=None):
     """g^T @ x, a layer's weight gradient over its input's rows, with the
     column sums of g (its bias gradient) in rowsum_out.  Split products where
     the weight has a 128 x 128 block for each of the 256 CUs, a vocabulary's
-    table above all: 50257 x 768 over 8192 rows takes 3.29 ms, 4.87 on the
+    table above all: 50257 x 768 over 8192 rows takes 3.6 ms, 4.87 on the
     float cores, over 2048 rows 0.90 and 1.38, and AdamW's g / (|g| + eps)
     makes of the changed roundings 2.8e-6 in GPT-2's second step's gradients
     (2-norm) and 2.4e-4 in single ones (of their root mean square).  Smaller
