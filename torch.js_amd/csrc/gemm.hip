@@ -616,7 +616,18 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs g, int splits) {
     float* out = const_cast<float*>(g.bias);
     for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < g.M; r += (int64_t)gridDim.x * 256) {
       float t = 0.f;
-      for (int q = 0; q < splits; ++q) t += g.rsw[q * g.M + r];
+      if (g.rs_pairs) {
+        Kahan k;
+        for (int q = 0; q < splits; ++q) {
+          const float x = g.rsw[2 * q * g.M + r];
+          t += x;
+          k.add(x);
+          k.add(g.rsw[(2 * q + 1) * g.M + r]);
+        }
+        if (t - t == 0.f) t = k.s - k.c;  // an infinity has no compensation
+      } else {
+        for (int q = 0; q < splits; ++q) t += g.rsw[q * g.M + r];
+      }
       out[r] = g.bias_mode == 3 ? t : out[r] + t;
     }
   }
@@ -906,6 +917,7 @@ int tjh::gemm(const char* family, int transA, int transB, int64_t M, int64_t N, 
   g.kchunk = BK;
   g.ws = nullptr;
   g.rsw = nullptr;
+  g.rs_pairs = 0;
   g.aux = act ? aux : nullptr;
   g.ldaux = ldaux;
   g.act = act;

@@ -34,6 +34,7 @@ struct GemmArgs {
   int64_t kchunk;  // K range per split (multiple of BK); splits = gridDim.y
   float* ws;       // split-K partials [batch][split][M][N] (nullptr: none)
   float* rsw;      // split-K partials of the row sums (bias_mode 3/4) [split][M]
+  int rs_pairs;    // 1: rsw is [split][2][M], each sum and what it rounds off
   // epilogue activation on the final C values (after alpha, beta, bias):
   // 1: aux (if any) <- v, C <- GELU(v);  2: C <- v * GELU'(aux);  3: C <- aux + v
   float* aux;

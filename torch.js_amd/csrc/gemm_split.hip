@@ -171,7 +171,7 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   g.kchunk = cdiv(cdiv(K, splits), BK) * BK;
   splits = cdiv(K, g.kchunk);
   // K slices: the products' partials, then the row sums'
-  const int64_t sums = bias_mode == 3 ? splits * M : 0;
+  const int64_t sums = bias_mode == 3 ? 2 * splits * M : 0;
   Scratch ws(splits > 1 ? (size_t)(splits * M * N + sums) * sizeof(float) : 0);
   if (splits > 1 && !ws.ok()) {
     splits = 1;
@@ -179,6 +179,7 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   }
   g.ws = splits > 1 ? ws.as<float>() : nullptr;
   g.rsw = splits > 1 && sums ? g.ws + splits * M * N : nullptr;
+  g.rs_pairs = 1;
   // tiles, K steps or loads that need a guard
   const bool edge = M % tc.bm || N % tc.bn || K % BK || !g.vecA || !g.vecB;
   launch_tile(plan.tile, g, dim3((unsigned)(g.tiles_m * g.tiles_n), (unsigned)splits), transA,
