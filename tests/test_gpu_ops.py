@@ -1248,6 +1248,26 @@ def test_attention_head_dims_about_the_short_products(torch, D, T, causal):
         check(got.numpy(), want, **RED)
 
 
+def test_attention_key_split_ends_with_the_causal_limit(torch):
+    """Causal queries over many more keys: the scratch for slices of the keys
+    goes as far as the queries see (three blocks of queries, 384 keys and 3
+    slices), not to the last key, and unseen keys don't matter."""
+    from torchjs_amd import _lib as L
+    r = np.random.default_rng(11)
+    H, Tq, Tk, D = 2, 300, 40000, 64
+    q, k, v = (f32(r.standard_normal((1, H, T, D))) for T in (Tq, Tk, Tk))
+    k[:, :, 5000:] = np.nan
+    t = [torch.tensor(a) for a in (q, k, v)]
+    L.check(L.lib().tjh_reset_peak())
+    before = torch.hip.memory_stats()["peak_bytes"]
+    with torch.no_grad():
+        y = torch.functional.scaled_dot_product_attention(*t, is_causal=True)
+        got = y.numpy()
+    used = torch.hip.memory_stats()["peak_bytes"] - before
+    assert used <= 8 * H * Tq * (D + 2) * 4  # the output, up to 3 slices, and rounding of blocks
+    check(got, _attend64(q, k[:, :, :Tq], v[:, :, :Tq], True), **RED)
+
+
 def test_attention_key_split_of_large_and_masked_scores(torch):
     """Scores of +-1e4 spread over the slices, and rows whose later slices
     underflow against the first."""

@@ -992,6 +992,13 @@ void launch_forward(const FlashArgs& a, unsigned grid) {
   else launch_forward_part<HD, false>(a, dim3(grid));
 }
 
+// Key tiles that some query sees: with `causal`, those up to the end of the
+// last block of queries.
+int64_t key_tiles(int64_t Tq, int64_t Tk, int causal) {
+  const int64_t end = cdiv(Tq, ROWS) * ROWS;
+  return cdiv(causal && end < Tk ? end : Tk, TILE);
+}
+
 // Key tiles per slice of a forward pass of BH heads, or 0 where its blocks
 // of ROWS queries fill the CUs by themselves.  A block walks its key tiles
 // one after the other, 2.6 us each, on one CU: 12 heads of 777 queries are 84
@@ -1000,7 +1007,7 @@ void launch_forward(const FlashArgs& a, unsigned grid) {
 // a CU: 27 + 6 us, 65 unsplit.
 int key_slice(int64_t BH, int64_t Tq, int64_t Tk, int causal) {
   const int64_t cus = num_cus() > 0 ? num_cus() : 256, blocks = cdiv(Tq, ROWS);
-  const int64_t nkt = cdiv(Tk, TILE);
+  const int64_t nkt = key_tiles(Tq, Tk, causal);
   if (BH * blocks >= cus || nkt <= 4) return 0;
   int64_t tiles = 0;
   for (int64_t i = 0; i < blocks; ++i) {
@@ -1080,7 +1087,7 @@ int flash_forward(const float* q, const float* k, const float* v, float* o, floa
   // slices of the keys only without lse: a recorded pass keeps its roundings
   const int64_t rows = B * H * Tq;
   a.kslice = lse ? 0 : key_slice(B * H, Tq, Tk, causal);
-  a.nsl = a.kslice ? (int)cdiv(cdiv(Tk, TILE), a.kslice) : 1;
+  a.nsl = a.kslice ? (int)cdiv(key_tiles(Tq, Tk, causal), a.kslice) : 1;
   Scratch part(a.nsl > 1 ? (size_t)(a.nsl * rows * (D + 2)) * sizeof(float) : 0);
   Scratch own_lse(!lse && !part.ok() ? (size_t)rows * sizeof(float) : 0);
   if (part.ok()) {
