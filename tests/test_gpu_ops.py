@@ -1248,6 +1248,20 @@ def test_attention_head_dims_about_the_short_products(torch, D, T, causal):
         check(got.numpy(), want, **RED)
 
 
+@pytest.mark.parametrize("H,T,causal", [(48, 400, False), (100, 200, True), (12, 130, True)])
+def test_attention_of_short_blocks_is_not_split(torch, H, T, causal):
+    """Where slices of the keys would not shorten the longest block by more
+    than the merge costs, a pass without a gradient is the recorded one, bit
+    for bit."""
+    r = np.random.default_rng(T)
+    q, k, v = (f32(r.standard_normal((1, H, T, 64))) for _ in range(3))
+    t = [torch.tensor(a, requires_grad=True) for a in (q, k, v)]
+    rec = torch.functional.scaled_dot_product_attention(*t, is_causal=causal).detach().numpy()
+    with torch.no_grad():
+        got = torch.functional.scaled_dot_product_attention(*t, is_causal=causal).numpy()
+    assert np.array_equal(got, rec)
+
+
 def test_attention_key_split_ends_with_the_causal_limit(torch):
     """Causal queries over many more keys: the scratch for slices of the keys
     goes as far as the queries see (three blocks of queries, 384 keys and 3

@@ -999,23 +999,31 @@ int64_t key_tiles(int64_t Tq, int64_t Tk, int causal) {
   return cdiv(causal && end < Tk ? end : Tk, TILE);
 }
 
-// Key tiles per slice of a forward pass of BH heads, or 0 where its blocks
-// of ROWS queries fill the CUs by themselves.  A block walks its key tiles
-// one after the other, 2.6 us each, on one CU: 12 heads of 777 queries are 84
+// Key tiles per slice of a forward pass of BH heads, or 0 where one workgroup
+// for a block of queries is as fast.  A block walks its key tiles one after
+// the other, 2.6 us each, on one CU: 12 heads of 777 queries are 84
 // workgroups, the longest of 25 tiles.  Slices of at least 4 tiles (fewer
-// spend as long on their prologue and on the merge) that make two workgroups
-// a CU: 27 + 6 us, 65 unsplit.
+// spend as long on their prologue) that make two workgroups a CU: 27 + 6 us,
+// 65 unsplit.  The merge takes as long as two to three tiles, and two
+// workgroups on a CU slow each other down, so the longest block has to be
+// longer than a slice by 3 tiles, or than two slices by 5 where some CUs get
+// two (over 309 shapes of 1 to 200 heads and 130 to 1024 keys no split then
+// loses more than 2%; 48 heads of 400 queries and keys 47 us split, 39
+// unsplit, 100 causal ones of 200 29 and 25, 12 of 130 20 and 17).
 int key_slice(int64_t BH, int64_t Tq, int64_t Tk, int causal) {
   const int64_t cus = num_cus() > 0 ? num_cus() : 256, blocks = cdiv(Tq, ROWS);
   const int64_t nkt = key_tiles(Tq, Tk, causal);
   if (BH * blocks >= cus || nkt <= 4) return 0;
-  int64_t tiles = 0;
-  for (int64_t i = 0; i < blocks; ++i) {
+  const auto ends = [&](int64_t i) {  // key tiles of query block i
     const int64_t end = (i + 1) * (ROWS / TILE);
-    tiles += causal && end < nkt ? end : nkt;
-  }
-  const int64_t s = cdiv(tiles * BH, 2 * cus);
-  return (int)(s < 4 ? 4 : s);
+    return causal && end < nkt ? end : nkt;
+  };
+  int64_t tiles = 0, groups = 0;
+  for (int64_t i = 0; i < blocks; ++i) tiles += ends(i);
+  int64_t s = cdiv(tiles * BH, 2 * cus);
+  if (s < 4) s = 4;
+  for (int64_t i = 0; i < blocks; ++i) groups += cdiv(ends(i), s);
+  return nkt < (groups * BH <= cus ? s + 3 : 2 * s + 5) ? 0 : (int)s;
 }
 
 // The key kernel (dK, dV) then the query kernel (dQ) of the backward; a.out
