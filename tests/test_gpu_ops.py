@@ -1191,6 +1191,31 @@ def test_few_rows_products(torch, M, N, K, shift):
     check(raw(alpha=s, bias=bias, bmode=1, act=1), ops.unary("gelu", s * z + bias), **RED)
 
 
+@pytest.mark.parametrize("ta,tb,M,N,K,split", [
+    (0, 1, 8, 256, 16384, False), (0, 1, 8, 1024, 64, False), (1, 0, 33, 256, 8192, False),
+    (0, 0, 64, 64, 2048, False), (0, 1, 4, 256, 16384, True), (0, 1, 8, 256, 8192, True),
+    (0, 0, 64, 1000, 768, True), (0, 0, 100, 256, 768, True), (0, 0, 128, 1024, 768, True),
+    (0, 0, 64, 256, 777, True)])
+def test_small_products_take_the_float_cores(torch, ta, tb, M, N, K, split):
+    """Small whole outputs and eight long or short rows are tjh_gemm's
+    products bit for bit; four rows, moderate K, ragged sides, K tails and 32
+    tiles are not."""
+    from torchjs_amd import _lib as L
+    r = np.random.default_rng(M + N + K)
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    a, b = (torch.tensor(np.ascontiguousarray(x.T) if t else x) for x, t in ((A, ta), (B, tb)))
+    c = torch.zeros(M, N)
+    L.check(L.lib().tjh_gemm(ta, tb, M, N, K, 1.0, a.data_ptr(), a.shape[1], 0, b.data_ptr(),
+                             b.shape[1], 0, 0.0, c.data_ptr(), N, 0, 1, None, 0))
+    flt = c.numpy().copy()
+    bias = f32(r.standard_normal(N))
+    got = _raw_split(torch, ta, tb, a.numpy(), b.numpy(), M, N, K)
+    assert np.array_equal(got, flt) != split
+    gelu = _raw_split(torch, ta, tb, a.numpy(), b.numpy(), M, N, K, alpha=1 / 64, bias=bias, bmode=1,
+                      act=1)
+    check(gelu, ops.unary("gelu", A.astype(np.float64) @ B.astype(np.float64) / 64 + bias), **RED)
+
+
 def _attend64(q, k, v, causal):
     q, k, v = (a.astype(np.float64) for a in (q, k, v))
     s = q @ k.swapaxes(-1, -2) / np.sqrt(q.shape[-1])

@@ -133,9 +133,23 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   TJH_ARG(lda >= (transA ? M : K) || (transA ? M : K) <= 1, "tjh_gemm_split: lda too small");
   TJH_ARG(ldb >= (transB ? K : N) || (transB ? K : N) <= 1, "tjh_gemm_split: ldb too small");
   TJH_ARG(ldc >= N, "tjh_gemm_split: ldc too small");
+  const int cus = num_cus() > 0 ? num_cus() : 256;
+  const bool aligned = (((uintptr_t)A | (uintptr_t)B) & 3) == 0;
+  // Few rows of A are multiplied where they are (gemm_rows.hip).  More than 4
+  // are more to read than B's rows once they leave the L1 (8 x 256 x 65536:
+  // 127 us, 47 on the float cores; x 8192: 10 and 16), and with short rows
+  // the sums over the lanes are most of the work (8 x 50257 x 64: 18 and 14).
+  const bool rows = !transA && transB && M <= kFewRows && K >= 32 && aligned && bias_mode != 3 &&
+                    cdiv(N, 4) < (int64_t(1) << 31) && (M <= 4 || (K >= 256 && K < 16384));
+  // An output of a few tiles is bound by the latency of its K steps, which
+  // are shorter on the float cores (64 x 256: 3 to 9% less time at 256 to
+  // 8192 terms, 9 x 256 x 32768 29 us and 35 to 41), except where they cut a
+  // ragged one into strips (64 x 1000: a third more).
+  const bool small = !rows && cdiv(M, 64) * cdiv(N, 64) < 32 && (M < 64 || M % 64 == 0) &&
+                     (N < 64 || N % 64 == 0) && K % BK == 0 && !getenv("TJH_SPLIT_TILE");
   // A^T . B^T and row sums of an A stored [M][K] have no kernel here, and
   // sums of fewer than two K steps nothing to gain: the float cores
-  if ((transA && transB) || (bias_mode == 3 && !transA) || K < 32) {
+  if (small || (transA && transB) || (bias_mode == 3 && !transA) || K < 32) {
     if (act == 1) {  // which keep the pre-activation
       Scratch keep((size_t)(M * N) * sizeof(float));
       if (!keep.ok()) return set_error(TJH_ERR_OOM, "tjh_gemm_split: no scratch");
@@ -145,7 +159,6 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
     return gemm("gemm", transA, transB, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 1,
                 bias, bias_mode, const_cast<float*>(residual), ldr, act);
   }
-  const int cus = num_cus() > 0 ? num_cus() : 256;
   GemmArgs g{};
   g.A = A; g.B = B; g.C = C; g.bias = bias;
   g.M = M; g.N = N; g.K = K;
@@ -157,9 +170,7 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   g.ldaux = ldr;
   g.act = act;
   KernelScope ks("gemm");
-  // few rows: nothing to gain from the matrix cores
-  if (!transA && transB && M <= kFewRows && g.vecA && g.vecB && cdiv(N, 4) < (int64_t(1) << 31))
-    return gemm_rows(g, cus);
+  if (rows) return gemm_rows(g, cus);
   const Plan plan = choose_plan(M, N, K, cus, transA);
   const TileCfg& tc = kTiles[plan.tile];
   g.tiles_m = (int)cdiv(M, tc.bm);
