@@ -1399,6 +1399,42 @@ def test_products_without_gradient_take_the_split_kernels(torch):
     check(z, y, **RED)
 
 
+@pytest.mark.parametrize("rows,out,inn,bias,split", [
+    (70, 32769, 128, True, True), (70, 32769, 128, False, True), (64, 5505, 768, True, True),
+    (70, 32640, 128, True, False), (64, 4096, 1024, True, False), (40, 4097, 1024, True, True),
+    (33, 1536, 2816, False, False), (64, 5120, 1280, True, False)])
+def test_weight_gradients_of_tables_are_split(torch, rows, out, inn, bias, split):
+    """Linear's gradients through backward(): split products for weights of
+    more than four rows to a column and 256 blocks of 128 x 128, the float
+    cores for every layer between others, whatever its width."""
+    from torchjs_amd import _lib as L
+    r = np.random.default_rng(out + inn)
+    x, w, b, g = (f32(r.standard_normal(s)) for s in ((rows, inn), (out, inn), (out,), (rows, out)))
+    tx, tw = torch.tensor(x, requires_grad=True), torch.tensor(w, requires_grad=True)
+    tb = torch.tensor(b, requires_grad=True) if bias else None
+    y = torch.functional.linear(tx, tw, tb)
+    real_lib, calls = L.lib(), []
+
+    class Spy:
+        def __getattr__(self, n):
+            return getattr(real_lib, n)
+
+        def tjh_gemm_split(self, *a):
+            calls.append(a[2:5])
+            return real_lib.tjh_gemm_split(*a)
+    try:
+        L._lib = Spy()
+        y.backward(torch.tensor(g))
+    finally:
+        L._lib = real_lib
+    assert calls == ([(out, inn, rows)] if split else [])
+    x8, w8, g8 = (a.astype(np.float64) for a in (x, w, g))
+    check_floor(tw.grad.numpy(), g8.T @ x8, g.T @ x)
+    check_floor(tx.grad.numpy(), g8 @ w8, g @ w)
+    if bias:
+        check_floor(tb.grad.numpy(), g8.sum(0), g.sum(0))
+
+
 def test_matmul_autograd_batched_broadcast(torch):
     r = np.random.default_rng(14)
     a = f32(r.standard_normal((2, 3, 4, 5)))

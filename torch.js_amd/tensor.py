@@ -2844,16 +2844,21 @@ def _gemm_ce(ce, b, trans):
 
 def _wgrad(g, x, rowsum_out=None):
     """g^T @ x, a layer's weight gradient over its input's rows, with the
-    column sums of g (its bias gradient) in rowsum_out.  Split products where
-    the weight has a 128 x 128 block for each of the 256 CUs, a vocabulary's
-    table above all: 50257 x 768 over 8192 rows takes 3.6 ms, 4.87 on the
-    float cores, over 2048 rows 0.90 and 1.38, and AdamW's g / (|g| + eps)
-    makes of the changed roundings 2.8e-6 in GPT-2's second step's gradients
-    (2-norm) and 2.4e-4 in single ones (of their root mean square).  Smaller
-    weights would gain as much (3072 x 768: 209 and 334 us), but theirs
-    become 9e-6 and 1.6e-3: the float cores."""
-    small = ((g._shape[1] + 127) // 128) * ((x._shape[1] + 127) // 128) < 256
-    return _gemm(g.T, x, rowsum_out=rowsum_out, recorded=small)
+    column sums of g (its bias gradient) in rowsum_out.  Split products for a
+    vocabulary's table: more than four rows to a column, wider than a layer
+    between others, and a 128 x 128 block for each of the MI355X's 256 CUs.
+    50257 x 768 over 8192 rows takes 3.6 ms, 4.87 on the float cores, over
+    2048 rows 0.90 and 1.38.  AdamW's g / (|g| + eps) carries the changed
+    roundings into the next step's gradients: 2.2e-6 of GPT-2's
+    (2-norm), 1.4e-4 of single ones (of their root mean square).  The
+    layers' weights would gain as much (3072 x 768: 232 and 334 us; 4096 x
+    1024: 0.37 and 0.57 ms), but move them by 5.6e-6 and 7.4e-4,
+    at widths of 1024 to 1536 by 6e-6 and 9e-4: the float cores.  (A
+    gradient of a cross-entropy that is not formed, under a seed other than
+    1, is multiplied on the float cores too: _gemm_ce.)"""
+    rows, cols = g._shape[1], x._shape[1]
+    table = rows > 4 * cols and ((rows + 127) // 128) * ((cols + 127) // 128) >= 256
+    return _gemm(g.T, x, rowsum_out=rowsum_out, recorded=not table)
 
 
 def _bgemm(a, b):
