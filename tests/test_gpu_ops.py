@@ -974,6 +974,20 @@ def test_gemm_split_row_sums_err_no_more_than_float(torch, M, N, K):
     assert split <= 1.01 * flt
 
 
+@pytest.mark.parametrize("M,N,K", [(4100, 1024, 65536), (50257, 768, 8192)])
+def test_gemm_split_scratch_of_tables(torch, M, N, K):
+    """The partials of a weight that fills the CUs take at most 12 times its
+    size (two rounds of the CUs in the widest tile), however many rows it is
+    summed over."""
+    from torchjs_amd import _lib as L
+    a, b, c = torch.zeros(K, M), torch.zeros(K, N), torch.zeros(M, N)
+    L.check(L.lib().tjh_reset_peak())
+    before = torch.hip.memory_stats()["peak_bytes"]
+    L.check(L.lib().tjh_gemm_split(1, 0, M, N, K, 1.0, a.data_ptr(), M, b.data_ptr(), N, 0.0,
+                                   c.data_ptr(), N, None, 0, None, 0, 0))
+    assert torch.hip.memory_stats()["peak_bytes"] - before <= 12 * 4 * M * N
+
+
 @pytest.mark.parametrize("tile", SPLIT_TILES)
 @pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0)])
 def test_gemm_split_not_finite_every_tile(torch, monkeypatch, tile, ta, tb):

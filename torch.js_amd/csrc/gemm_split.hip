@@ -74,7 +74,10 @@ Plan choose_plan(int64_t M, int64_t N, int64_t K, int cus, bool ta) {
   const int64_t slice = 2 * blocks < cus ? 512 : blocks < 2 * cus ? 2048 : K + 1;
   int64_t smax = K / 64 < 64 ? K / 64 : 64;
   if (smax < 1) smax = 1;
-  const int64_t smin = cdiv(K, slice) < smax ? cdiv(K, slice) : smax;
+  int64_t smin = cdiv(K, slice) < smax ? cdiv(K, slice) : smax;
+  // no more than the float cores' most for an output that fills the CUs: the
+  // partials of 4100 x 1024 over 65536 terms stay at 134 MB (32 slices: 537)
+  if (blocks >= cus && smin > 8) smin = 8;
   Plan best{kNumTiles - 1, 1};
   double best_t = 1e300;
   for (int i = 0; i < kNumTiles; ++i) {
