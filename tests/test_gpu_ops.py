@@ -1183,6 +1183,53 @@ def test_gemm_split_error_of_scaled_operands(torch, scale):
     assert np.linalg.norm(got - want) <= 4.8e-7 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("tile", SPLIT_TILES)
+@pytest.mark.parametrize("ta,tb,K,scale", [(0, 1, 300, 1), (1, 0, 512, 2.0 ** 60), (0, 0, 6000, 1)])
+def test_gemm_split_tiny_operands_every_tile(torch, monkeypatch, tile, ta, tb, K, scale):
+    """Operands under 2^-109 lose bits of their parts: rows of 2^-112 to
+    2^-130, subnormal ones among them, beside a row of ordinary values and
+    tiny ones mixed, are no further off 64 bits than the float cores'
+    products."""
+    from torchjs_amd import _lib as L
+    monkeypatch.setenv("TJH_SPLIT_TILE", tile)
+    r = np.random.default_rng(K)
+    M, N = 280, 90
+    e = np.full(M, -112.0)
+    e[64:], e[128:], e[160:], e[200:] = -118, -126, -130, 0
+    A = f32(r.standard_normal((M, K)) * 2.0 ** e[:, None])
+    A[200:, ::7] *= f32(2.0 ** -120)
+    A[210, :] = 0
+    B = f32(r.standard_normal((K, N)) * scale)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    got = _raw_split(torch, ta, tb, np.ascontiguousarray(A.T) if ta else A,
+                     np.ascontiguousarray(B.T) if tb else B, M, N, K)
+    a, b = (torch.tensor(np.ascontiguousarray(x.T) if t else x) for x, t in ((A, ta), (B, tb)))
+    c = torch.zeros(M, N)
+    L.check(L.lib().tjh_gemm(ta, tb, M, N, K, 1.0, a.data_ptr(), a.shape[1], 0, b.data_ptr(),
+                             b.shape[1], 0, 0.0, c.data_ptr(), N, 0, 1, None, 0))
+    flt = c.numpy()
+    for x in np.unique(e):
+        rows = e == x
+        # a sum of K terms in one slice errs at most sqrt(K / 2) roundings'
+        # root mean square, 0.29 of 2^-23, and one of a subnormal result
+        floor = 0.29 * 2.0 ** -23 * np.sqrt(K / 2) * np.linalg.norm(want[rows]) + \
+            2.0 ** -149 * np.sqrt(want[rows].size)
+        assert np.linalg.norm(got[rows] - want[rows]) <= max(np.linalg.norm(flt[rows] - want[rows]), floor)
+    assert not got[210].any() and not np.signbit(got[210]).any()
+
+
+def test_gemm_split_tiny_operands_leave_ordinary_sums(torch):
+    """Where a few tiny operands don't touch the sums, the product is the
+    split one: its bits don't change when they are set to zero."""
+    r = np.random.default_rng(4)
+    M, N, K = 300, 260, 200
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    A[::3, 5] = f32(2.0 ** -120) * A[::3, 5]
+    got = _raw_split(torch, 0, 0, A, B, M, N, K)
+    A[::3, 5] = 0
+    assert np.array_equal(got, _raw_split(torch, 0, 0, A, B, M, N, K))
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 7, 8, 9])
 @pytest.mark.parametrize("N,K,shift", [(1, 33, 0), (770, 768, 0), (2049, 1001, 1), (8200, 40, 2),
                                        (65, 3071, 3)])

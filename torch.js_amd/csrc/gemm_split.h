@@ -64,6 +64,9 @@
 
 #include "gemm_args.h"
 #include "kahan.h"
+#include "wave.h"
+
+#include <math.h>
 
 namespace tjh {
 
@@ -72,8 +75,9 @@ namespace tjh {
 // A float as three bfloat16 parts: x = h + m + l, each part the nearest
 // bfloat16 of what is left.  Three times eight significant bits hold the 24
 // of a float: the sum is exact while the parts stay above the smallest
-// bfloat16 (2^-133), so for |x| >= 2^-109; below, an absolute error of at
-// most 2^-134 remains.  For 1 <= |x| < 2, |m| <= 2^-8 and |l| <= 2^-17, so
+// bfloat16 (2^-133; the matrix cores keep subnormal operands), so for |x| >=
+// 2^-109; below, an absolute error of at most 2^-134 remains (tiny_operand).
+// For 1 <= |x| < 2, |m| <= 2^-8 and |l| <= 2^-17, so
 // of the nine products of two split numbers the three not formed (m l, l m,
 // l l) are at most 2^-24 + 2^-34 of the product, one float rounding of it
 // (a tenth of that in the root mean square over normal values).
@@ -203,8 +207,9 @@ struct Tile {
     }
   }
   // Splits the tile and stores its parts in LDS, `part` bytes apart, outer
-  // index o negated where o + flip is odd (kFlip below).
-  __device__ __forceinline__ void store(char* __restrict__ S, int part) const {
+  // index o negated where it is odd.  `top` is raised to the largest
+  // magnitude.
+  __device__ __forceinline__ void store(char* __restrict__ S, int part, float& top) const {
 #pragma unroll
     for (int i = 0; i < I; ++i) {
       if (!has(i)) continue;
@@ -217,6 +222,8 @@ struct Tile {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           unsigned a, b, c;
+          // (fmaxf would first quiet each operand)
+          asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(r[i][w][2 * q]), "v"(r[i][w][2 * q + 1]));
           split2(r[i][w][2 * q], r[i][w][2 * q + 1], sign, a, b, c);
           h[q] = a;
           m[q] = b;
@@ -247,6 +254,23 @@ __device__ __forceinline__ int xcd_tile(int bid, int n) {
 // SIMD (256 registers each), smaller ones three or more.
 constexpr int gemm_waves_per_simd(int wm, int wn) {
   return wm * wn >= 64 * 64 ? 2 : wm * wn >= 64 * 32 ? 3 : 4;
+}
+
+// Whether outer index o (clamped to n) of an operand, stored [k][outer] (KT)
+// or [outer][k], has a value but zero under 2^-109 among its k = kbeg + h,
+// + 2, ...
+template <bool KT>
+__device__ __forceinline__ bool tiny_operand(const float* __restrict__ P, int64_t ld, int64_t o,
+                                             int64_t n, int h, int64_t kbeg, int64_t kend) {
+  if (o >= n) o = n - 1;
+  const float* __restrict__ p = KT ? P + o : P + o * ld;
+  bool tiny = false;
+#pragma unroll 4
+  for (int64_t k = kbeg + h; k < kend; k += 2) {
+    const float x = __builtin_fabsf(p[KT ? k * ld : k]);
+    tiny |= x > 0.f && x < 0x1p-109f;
+  }
+  return tiny;
 }
 
 // The 32 x 32 block of products over [kbeg, kend) that holds row `row` (of
@@ -297,6 +321,7 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   constexpr int PA = BM * BK * 2, PB = BN * BK * 2, BUF = 3 * (PA + PB);
   static_assert(FM >= 1 && FN >= 1 && FM * 32 == WM && FN * 32 == WN, "tile");
   __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
+  __shared__ float tops[WR * WC];  // each wave's largest operand
 
   // Wave priority: the prologue and the epilogue run at raised priority.
   // Where two workgroups share a CU, at equal priority the one in its
@@ -359,11 +384,12 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
     xa.load(A, g.lda, g.M, m0, k0);
     xb.load(B, g.ldb, g.N, n0, k0);
   };
+  float top = 0.f;
   auto stage = [&](int64_t t, TileA& xa, TileB& xb) {
     char* S = lds + (t & 1) * BUF;
     if (TA && row_sums) xa.sum(rsum);
-    xa.store(S, PA);
-    xb.store(S + 3 * PA, PB);
+    xa.store(S, PA, top);
+    xb.store(S + 3 * PA, PB, top);
   };
   // the six products of a K tile, the smallest terms first
   auto compute = [&](int64_t t) {
@@ -449,6 +475,9 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   }
 
   __builtin_amdgcn_s_setprio(3);
+  top = wave_max(top);
+  if (lane == 0) tops[wid] = top;
+  __syncthreads();
   if (TA && row_sums) {
     // the two k halves of a row are in two lanes, added with what their
     // compensations hold (50257 rows over 8192: 3.9e-8 off 64 bits, 5.6e-8 by
@@ -522,6 +551,14 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   // float arithmetic.  0 * x is 0 for finite x and NaN otherwise.  2048 x
   // 3072 x 768 takes 75 us, with a NaN in every row 243 us (11.3 ms by
   // multiply-adds one after the other, 89 us on gemm.hip's tiles).
+  // Operands under 2^-109, too: what the parts lose of them is 2^-134 a term
+  // times the other operand, which only sums under `least` can show; a block
+  // that has such a sum looks for such operands.  (Following the largest
+  // operand for it costs 1.5% of a large product.)
+  float least = 0.f;
+#pragma unroll
+  for (int w = 0; w < WR * WC; ++w) least = fmaxf(least, tops[w]);
+  least *= (float)(kend - kbeg) * 0x1p-108f;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -532,9 +569,17 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
         z0 = __builtin_fmaf(acc[i][j][r], 0.f, z0);
         z1 = __builtin_fmaf(acc[i][j][r + 1], 0.f, z1);
       }
-      if (__any(!(z0 + z1 == 0.f))) {
-        acc[i][j] = float_block<TA, TB>(g, m0 + wm * WM + i * 32 + l32, n0 + wn * WN + j * 32 + l32,
-                                        h, kbeg, kend);
+      bool again = !(z0 + z1 == 0.f);
+      const int64_t row = m0 + wm * WM + i * 32 + l32, col = n0 + wn * WN + j * 32 + l32;
+      float least_sum = INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; r += 2)
+        asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least_sum) : "v"(acc[i][j][r]), "v"(acc[i][j][r + 1]));
+      if (__any(least_sum < least))
+        again |= tiny_operand<TA>(g.A, g.lda, row, g.M, h, kbeg, kend) ||
+                 tiny_operand<!TB>(g.B, g.ldb, col, g.N, h, kbeg, kend);
+      if (__any(again)) {
+        acc[i][j] = float_block<TA, TB>(g, row, col, h, kbeg, kend);
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] *= r & 1 ? -sign : sign;
       }
