@@ -9,13 +9,15 @@ next-token cross_entropy; full backward; AdamW(lr 6e-4, wd 0.1).
 
 Prints ONE JSON line.  `value` = tokens/s over exactly K timed steps
 (inputs resident in HBM, device synchronised on both sides of the timed
-region).  `roofline` reports the dominant kernel family (the MFMA GEMMs of
+region).  `roofline` reports the dominant kernel family (the fp32 MFMA GEMMs of
 the Linear layers) from the start / stop timestamps of each of its
 kernels' own dispatches (hipExtLaunchKernel events: no marker packets
 between launches) over K more steps right after the timed region, the
 same work (the timestamps cost ~10 us of issue time per launch, so they
-stay out of the region that gives `value`); `roofline.traffic` is the HBM bytes
-per launch measured by rocprofv3 counters
+stay out of the region that gives `value`); `roofline.table_wgrad` is the one
+product of the step on the bf16 matrix cores, from the per-kernel pass, against
+a sixth of their peak; `roofline.traffic` is the HBM bytes per launch
+measured by rocprofv3 counters
 (profiles/gemm_hbm_traffic_gpt2.json).  `hbm_kernels` and
 `kernel_ms_per_step` come from a pass after the timed region in which
 every kernel carries such timestamps (the sums are kernel execution time,
@@ -44,9 +46,11 @@ sys.path.insert(0, ROOT)
 
 METRIC = "GPT-2 124M fwd+bwd+AdamW tokens/s (1 GPU); bwd-kernel HBM GB/s vs peak"
 HBM_PEAK_GBS = 8000.0
-DOMINANT = "gemm"  # kernel family of the Linear-layer GEMMs (k_gemm + split-K reduce)
+DOMINANT = "gemm"  # kernel family of the fp32 MFMA GEMMs (k_gemm + split-K reduce)
+SPLIT = "gemm_split"  # floats as three bf16 parts: the token table's weight gradient
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "gemm_hbm_traffic_gpt2.json")
 FP32_MFMA_PEAK_TFLOPS = 157.3
+BF16_MFMA_PEAK_TFLOPS = 2500.0  # dense
 
 V, CTX, D, H, LAYERS = 50257, 1024, 768, 12, 12
 B, T = 8, 1024
@@ -554,15 +558,24 @@ def main():
     ms_step = 1000.0 * elapsed / args.steps
     # dominant kernel: the Linear GEMMs (MFMA), timed inside the timed region
     n_g, ms_g = dominant
-    flops = linear_flops_per_step(B, T) * args.steps
+    n_s, ms_s = timing.get(SPLIT, (0, 0.0))
+    table_flops = 2 * B * T * V * D if ms_s else 0
+    flops = (linear_flops_per_step(B, T) - table_flops) * args.steps
     achieved = flops / (ms_g / 1000.0) / 1e12 if ms_g else 0.0
-    roofline = {"bound": "mfma", "kernel": "k_gemm family (Linear fwd/dgrad/wgrad + LM head, "
-                "fp32 MFMA, incl. split-K reduce)",
+    roofline = {"bound": "mfma", "kernel": "k_gemm family (Linear fwd/dgrad/wgrad, LM "
+                "head fwd/dgrad; fp32 MFMA, incl. split-K reduce)",
                 "achieved": round(achieved, 2), "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4), "traffic": traffic_per_launch(),
                 "launches": n_g, "avg_launch_ms": round(ms_g / max(n_g, 1), 4),
                 "flop_per_launch": round(flops / max(n_g, 1)),
                 "share_of_step": round(ms_g / (ms_step * args.steps), 3)}
+    if ms_s:
+        # six bf16 products for each float one
+        rate = table_flops * prof_steps / (ms_s / 1000.0) / 1e12
+        roofline["table_wgrad"] = {"kernel": "k_gemm_split (LM head wgrad, 6 bf16 MFMA products)",
+                                   "achieved": round(rate, 2), "peak": round(BF16_MFMA_PEAK_TFLOPS / 6, 1),
+                                   "unit": "TFLOP/s", "frac": round(6 * rate / BF16_MFMA_PEAK_TFLOPS, 4),
+                                   "ms_per_step": round(ms_s / prof_steps, 3)}
     hbm = {}
     for fam, byts in hbm_bytes_per_step(B, T, nparams, distinct).items():
         n, ms = timing.get(fam, (0, 0.0))

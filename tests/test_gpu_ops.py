@@ -1496,6 +1496,23 @@ def test_weight_gradients_of_tables_are_split(torch, rows, out, inn, bias, split
         check_floor(tb.grad.numpy(), g8.sum(0), g.sum(0))
 
 
+def test_split_products_are_timed_apart(torch):
+    """Split products, few-row ones and the float cores' are families of
+    their own in the kernel timing."""
+    a, b = torch.zeros(256, 128), torch.zeros(1000, 128)
+    try:
+        torch.hip.kernel_timing(True)
+        torch.hip.kernel_timing_reset()
+        with torch.no_grad():
+            torch.functional.linear(a, b)
+            torch.functional.linear(a[:2], b)
+        torch.functional.linear(a, torch.tensor(b.numpy(), requires_grad=True))
+        counts = [torch.hip.kernel_time(f)[0] for f in ("gemm_split", "gemm_rows", "gemm")]
+    finally:
+        torch.hip.kernel_timing(False)
+    assert counts[:2] == [1, 1] and counts[2] > 0
+
+
 def test_matmul_autograd_batched_broadcast(torch):
     r = np.random.default_rng(14)
     a = f32(r.standard_normal((2, 3, 4, 5)))

@@ -172,7 +172,7 @@ extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int6
   g.aux = act == 3 ? const_cast<float*>(residual) : nullptr;
   g.ldaux = ldr;
   g.act = act;
-  KernelScope ks("gemm");
+  KernelScope ks(rows ? "gemm_rows" : "gemm_split");
   if (rows) return gemm_rows(g, cus);
   const Plan plan = choose_plan(M, N, K, cus, transA);
   const TileCfg& tc = kTiles[plan.tile];
