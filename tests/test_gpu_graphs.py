@@ -125,6 +125,35 @@ def test_graph_memory_is_not_shared_with_eager_work(torch):
     g.reset()
 
 
+def test_inference_replays_like_eager_calls(torch):
+    """A prompt and a cached token without gradients, with K slices, slices of
+    the keys and the few-row products among their launches, captured and
+    replayed with other inputs between eager passes, equal the eager calls."""
+    from torchjs_amd import workloads as W
+    m = W.GPT2(vocab=211, ctx=320, d=128, heads=2, layers=2)
+    r = np.random.default_rng(3)
+    ids = [torch.tensor(r.integers(0, 211, (2, 300)).astype(np.int32)) for _ in range(3)]
+    tok = [torch.tensor(r.integers(0, 211, (2, 1)).astype(np.int32)) for _ in range(3)]
+    with torch.no_grad():
+        caches = [m.new_cache(2) for _ in range(4)]
+        want = [(m.forward_cached(a, c, 0).numpy(), m.forward_cached(b, c, 300).numpy())
+                for a, b, c in zip(ids, tok, caches)]
+        a, b = torch.zeros(2, 300, dtype="int32"), torch.zeros(2, 1, dtype="int32")
+        g = torch.hip.Graph()
+        with torch.hip.graph(g):
+            y = m.forward_cached(a, caches[3], 0)
+            z = m.forward_cached(b, caches[3], 300)
+        for i in (0, 1, 2, 0):
+            a.copy_(ids[i])
+            b.copy_(tok[i])
+            g.replay()
+            _bits(y.numpy(), want[i][0])
+            _bits(z.numpy(), want[i][1])
+            m(ids[2])  # eager work between the replays
+            torch.synchronize()
+    g.reset()
+
+
 def test_readback_inside_capture_raises(torch):
     x = torch.tensor(_rand((256, 256), 41))
     g = torch.hip.Graph()

@@ -1430,6 +1430,25 @@ def test_block_without_gradient_is_one_call(torch, monkeypatch, B, T, C, heads):
     assert len(calls) == n
 
 
+def test_block_without_gradient_heeds_what_a_program_replaces(torch):
+    """Methods replaced on a block's layers or on the cache lead to the layers
+    one by one."""
+    from torchjs_amd import workloads as W
+    blk = W.Block(64, 2)
+    x = torch.tensor(f32(np.random.default_rng(1).standard_normal((2, 5, 64))))
+    with torch.no_grad():
+        want = blk(x).numpy()
+        plain = blk.attn._project
+        blk.attn._project = lambda y, residual: plain(y, residual) + 1.0
+        assert np.abs(blk(x).numpy() - want).max() > 0.1
+        del blk.attn.__dict__["_project"]
+        cache, seen = W.KVCache(1, 2, 2, 8, 32), []
+        append = cache.append
+        cache.append = lambda *a: seen.append(a[3]) or append(*a)
+        np.testing.assert_array_equal(blk.forward_cached(x, cache, 0, 0).numpy(), want)
+        assert seen == [0]
+
+
 def test_products_without_gradient_take_the_split_kernels(torch):
     """Linear, the residual and MLP forms and matmul: split products exactly
     where nothing is recorded, equal to the recorded ones within rounding."""

@@ -150,7 +150,7 @@ class Block(nn.Module):
         if not (tuple(map(type, mods)) == _BLOCK_MODULES and at.fused and mlp.fused and
                 x.ndim == 3 and x.dtype == "float32"):
             return None
-        if any("forward" in m.__dict__ or "forward_cached" in m.__dict__ for m in mods):
+        if any(k in m.__dict__ for m in mods for k in ("forward", "forward_cached", "_project")):
             return None
         B, T, C = x.shape
         hd, hid = C // at.heads, mlp.c_fc.weight.shape[0]
@@ -173,7 +173,8 @@ class Block(nn.Module):
         kc = vc = None
         max_len = 0
         if cache is not None:
-            if type(cache) is not KVCache or pos < 0 or (pos and T != 1):
+            if type(cache) is not KVCache or "append" in cache.__dict__ or pos < 0 or \
+                    (pos and T != 1):
                 return None
             kc, vc = cache.k[layer], cache.v[layer]
             max_len = cache.max_len
