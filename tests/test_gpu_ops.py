@@ -1430,10 +1430,10 @@ def test_block_without_gradient_is_one_call(torch, monkeypatch, B, T, C, heads):
     assert len(calls) == n
 
 
-def test_block_without_gradient_heeds_what_a_program_replaces(torch):
-    """Methods replaced on a block's layers or on the cache lead to the layers
-    one by one."""
-    from torchjs_amd import workloads as W
+def test_block_without_gradient_heeds_what_a_program_replaces(torch, monkeypatch):
+    """Methods replaced on a block's layers or on the cache, and a workspace
+    that does not fit, lead to the layers one by one."""
+    from torchjs_amd import _lib as L, workloads as W
     blk = W.Block(64, 2)
     x = torch.tensor(f32(np.random.default_rng(1).standard_normal((2, 5, 64))))
     with torch.no_grad():
@@ -1447,6 +1447,13 @@ def test_block_without_gradient_heeds_what_a_program_replaces(torch):
         cache.append = lambda *a: seen.append(a[3]) or append(*a)
         np.testing.assert_array_equal(blk.forward_cached(x, cache, 0, 0).numpy(), want)
         assert seen == [0]
+        real = L.lib()
+
+        class NoRoom:
+            def __getattr__(self, n):
+                return (lambda *a: L.ERR_OOM) if n == "tjh_block_infer" else getattr(real, n)
+        monkeypatch.setattr(L, "_lib", NoRoom())
+        np.testing.assert_array_equal(blk(x).numpy(), want)
 
 
 def test_products_without_gradient_take_the_split_kernels(torch):

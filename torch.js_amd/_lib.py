@@ -252,6 +252,9 @@ def lib():
 ERR_UNSUPPORTED = 5  # TJH_ERR_UNSUPPORTED
 
 
+ERR_OOM = 3  # TJH_ERR_OOM
+
+
 def check(rc, what=""):
     if rc != 0:
         msg = lib().tjh_last_error()

@@ -191,11 +191,14 @@ class Block(nn.Module):
         if cache is not None:
             _before_write(kc, vc)
         y = empty((B, T, C))
-        L.check(L.lib().tjh_block_infer(
+        rc = L.lib().tjh_block_infer(
             px, y.data_ptr(), (ctypes.c_void_p * 12)(*w), B, T, C, at.heads, hid,
             float(self.ln_1.eps), float(self.ln_2.eps), 1.0 / math.sqrt(hd),
             kc.data_ptr() if kc is not None else None, vc.data_ptr() if vc is not None else None,
-            max_len, pos), "block_infer")
+            max_len, pos)
+        if rc == L.ERR_OOM:  # no room for the workspace in one piece
+            return None
+        L.check(rc, "block_infer")
         return y
 
     def forward_cached(self, x, cache, layer, pos):
