@@ -893,14 +893,29 @@ SPLIT_TILES = ["256x128", "128x128", "128x64", "64x64"]
 
 
 @pytest.mark.parametrize("tile", SPLIT_TILES)
-@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K,shift", [(300, 260, 200, 0), (256, 384, 4096, 0), (5, 3, 35, 1),
-                                         (257, 193, 541, 3), (130, 129, 31, 0)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+@pytest.mark.parametrize("M,N,K,shift", [(300, 260, 200, 0), (256, 384, 4096, 0), (9, 3, 35, 1),
+                                         (257, 193, 541, 3), (130, 129, 32, 0)])
 def test_gemm_split_every_tile(torch, monkeypatch, tile, ta, tb, M, N, K, shift):
     """Whole tiles, tiles over both edges, K tails, slices of K, operands off
-    16-byte alignment, and the products left to the float cores (K < 32,
-    both operands transposed)."""
+    16-byte alignment."""
     monkeypatch.setenv("TJH_SPLIT_TILE", tile)
+    r = np.random.default_rng(M + N + K + ta * 2 + tb)
+    A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
+    bias, C0 = f32(r.standard_normal(N)), f32(r.standard_normal((M, N)))
+    want = 0.5 * (A.astype(np.float64) @ B.astype(np.float64)) + 0.25 * C0 + bias
+    got = _raw_split(torch, ta, tb, np.ascontiguousarray(A.T) if ta else A,
+                     np.ascontiguousarray(B.T) if tb else B, M, N, K, 0.5, 0.25, C0, bias, 1,
+                     shift=shift)
+    check_floor(got, want, np.float32(0.5) * (A @ B) + np.float32(0.25) * C0 + bias)
+
+
+@pytest.mark.parametrize("ta,tb,M,N,K,shift", [(1, 1, 300, 260, 200, 0), (1, 1, 257, 193, 541, 3),
+                                               (0, 0, 130, 129, 31, 0), (0, 1, 130, 129, 31, 1),
+                                               (1, 0, 130, 129, 1, 0), (0, 1, 5, 3, 35, 1)])
+def test_gemm_split_left_to_other_kernels(torch, ta, tb, M, N, K, shift):
+    """Products that have no split kernel: both operands transposed and K <
+    32 on the float cores, few rows on their own kernel."""
     r = np.random.default_rng(M + N + K + ta * 2 + tb)
     A, B = f32(r.standard_normal((M, K))), f32(r.standard_normal((K, N)))
     bias, C0 = f32(r.standard_normal(N)), f32(r.standard_normal((M, N)))
@@ -1056,6 +1071,29 @@ def test_gemm_split_zeros_are_positive_every_tile(torch, monkeypatch, tile, ta, 
                      np.ascontiguousarray(B.T) if tb else B, M, N, K)
     assert (got[:192] == 0).all() and (got[:, 60:] == 0).all()
     assert not np.signbit(got[got == 0]).any()
+
+
+@pytest.mark.parametrize("K", [70, 6001])
+def test_gemm_split_not_finite_row_sums(torch, K):
+    """A weight gradient whose gradient holds an infinity and a NaN: their
+    rows' sums are not finite, the others' keep their values."""
+    from torchjs_amd import _lib as L
+    r = np.random.default_rng(K)
+    M, N = 300, 70
+    A, B = f32(r.standard_normal((K, M))), f32(r.standard_normal((K, N)))
+    A[5, 7], A[K - 1, 130], A[3, 299] = np.inf, np.nan, -np.inf
+    a, b, c, s = torch.tensor(A), torch.tensor(B), torch.zeros(M, N), torch.zeros(M)
+    L.check(L.lib().tjh_gemm_split(1, 0, M, N, K, 1.0, a.data_ptr(), M, b.data_ptr(), N, 0.0,
+                                   c.data_ptr(), N, s.data_ptr(), 3, None, 0, 0))
+    bad = np.zeros(M, bool)
+    bad[[7, 130, 299]] = True
+    s, c = s.numpy(), c.numpy()
+    assert np.array_equal(~np.isfinite(s), bad)
+    assert np.isnan(s[130]) and np.isnan(c[130]).all()
+    assert np.array_equal(c[7], np.where(B[5] > 0, np.inf, -np.inf))
+    want = A[:, ~bad].astype(np.float64)
+    check_floor(c[~bad], want.T @ B.astype(np.float64), A[:, ~bad].T @ B)
+    assert np.abs(s[~bad] - want.sum(0)).max() <= 2 ** -23 * np.abs(want.sum(0)).max()
 
 
 def test_gemm_split_not_finite_costs_a_float_product(torch):
@@ -1303,12 +1341,37 @@ def test_attention_of_few_workgroups(torch, D, Tq, Tk, causal):
         tk, tv = (torch.tensor(a)[:, :, :Tk] for a in (k, v))
         got = torch.functional.scaled_dot_product_attention(torch.tensor(q), tk, tv,
                                                             is_causal=causal).numpy()
-    # the recorded form: one workgroup for all keys of 128 queries
-    tq = torch.tensor(q, requires_grad=True)
-    rec = torch.functional.scaled_dot_product_attention(tq, tk, tv, is_causal=causal).detach().numpy()
     want = _attend64(q, k[:, :, :Tk], v[:, :, :Tk], causal)
     check(got, want, **RED)
-    assert np.linalg.norm(got - want) <= 1.5 * np.linalg.norm(rec - want) + 1e-7 * np.linalg.norm(want)
+    # the recorded form: one workgroup for all keys of 128 queries (of one
+    # query it is the same kernel)
+    tq = torch.tensor(q, requires_grad=True)
+    rec = torch.functional.scaled_dot_product_attention(tq, tk, tv, is_causal=causal).detach().numpy()
+    if Tq == 1:
+        assert np.array_equal(got, rec)
+    else:
+        assert np.linalg.norm(got - want) <= 1.02 * np.linalg.norm(rec - want)
+
+
+@pytest.mark.parametrize("D", [4, 40, 64, 128])
+@pytest.mark.parametrize("Tk,causal", [(1, False), (7, True), (64, False), (701, False)])
+def test_attention_gradients_of_one_query(torch, D, Tk, causal):
+    """The lse that the one-query kernel keeps serves the backward kernels."""
+    r = np.random.default_rng(D + Tk)
+    q, g = (f32(r.standard_normal((2, 3, 1, D))) for _ in range(2))
+    k, v = (f32(r.standard_normal((2, 3, Tk, D))) for _ in range(2))
+    t = [torch.tensor(a, requires_grad=True) for a in (q, k, v)]
+    torch.functional.scaled_dot_product_attention(*t, is_causal=causal).backward(torch.tensor(g))
+    q, k, v, g = (a.astype(np.float64) for a in (q, k, v, g))
+    s = q @ k.swapaxes(-1, -2) / np.sqrt(D)
+    if causal:
+        s[..., 1:] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    dp = g @ v.swapaxes(-1, -2)
+    ds = p * (dp - (p * dp).sum(-1, keepdims=True)) / np.sqrt(D)
+    for got, want in zip([a.grad for a in t], [ds @ k, ds.swapaxes(-1, -2) @ q, p.swapaxes(-1, -2) @ g]):
+        check(got.numpy(), want, **RED)
 
 
 @pytest.mark.parametrize("D", [4, 16, 20, 40, 48, 52, 80, 84, 112, 116])
