@@ -21,16 +21,9 @@
 #include <float.h>
 
 namespace tjh {
-
-// attn_one.hip
-int attn_one_query(const float* q, const float* k, const float* v, float* o, float* lse, int64_t B,
-                   int64_t H, int64_t Tk, int64_t D, const int64_t* qs, const int64_t* ks,
-                   const int64_t* vs, const int64_t* os, float scale, int causal);
-
 namespace {
 
 constexpr int kBlock = 256;
-
 
 // In place: S (already scaled) -> P, lse[row] written.  Row r of [H*Tq]
 // has query index i = r % Tq; with causal only cols j <= i are valid.

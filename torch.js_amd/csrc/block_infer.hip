@@ -35,11 +35,6 @@ __global__ __launch_bounds__(256) void k_kv_append(const float* __restrict__ qkv
 
 using namespace tjh;
 
-extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,
-                              const float* A, int64_t lda, const float* B, int64_t ldb, float beta,
-                              float* C, int64_t ldc, const float* bias, int bias_mode,
-                              const float* residual, int64_t ldr, int act);
-
 /* y = x1 + MLP(LN2(x1)), x1 = x + proj(attention(qkv(LN1(x)))) for x, y
  * [B, T, C], contiguous.  w: ln1 weight, bias, qkv weight, bias, proj weight,
  * bias, ln2 weight, bias, fc weight, bias, fc2 weight, bias (weights [out,

@@ -108,6 +108,12 @@ int flash_backward(const float* q, const float* k, const float* v, const float* 
                    int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t D,
                    const int64_t* const* strides, float scale, int causal);
 
+// Attention of one query a head, for the layouts of flash_supported
+// (attn_one.hip); lse may be null.
+int attn_one_query(const float* q, const float* k, const float* v, float* o, float* lse, int64_t B,
+                   int64_t H, int64_t Tk, int64_t D, const int64_t* qs, const int64_t* ks,
+                   const int64_t* vs, const int64_t* os, float scale, int causal);
+
 // 16-byte alignment of a device pointer (128-bit access paths).
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -129,6 +135,21 @@ __device__ __forceinline__ void st_nt(float* p, const float4& v) {
 __host__ __device__ inline int64_t cdiv(int64_t n, int64_t d) { return (n + d - 1) / d; }
 
 }  // namespace tjh
+
+/* tjh_gemm (batch 1) for a result that no gradient is taken through: float
+ * products formed from three bf16 parts of each operand (gemm_split.h), or
+ * for few rows multiply-adds (gemm_rows.hip), or tjh_gemm's own where they
+ * gain nothing.  Its error against 64 bits is no larger than tjh_gemm's, but
+ * its roundings are others.
+ * act 0: nothing; 1: C = GELU(v); 3: C = residual + v, with residual [M][N]
+ * at row stride ldr, not overlapping C.  bias_mode 0 to 3 as tjh_gemm, 3
+ * (bias receives the row sums of op(A)) with act 0 only.
+ * For the Python host, which knows what is recorded; not part of the
+ * library's declared interface. */
+extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,
+                              const float* A, int64_t lda, const float* B, int64_t ldb, float beta,
+                              float* C, int64_t ldc, const float* bias, int bias_mode,
+                              const float* residual, int64_t ldr, int act);
 
 #define TJH_REQUIRE_INIT()                   \
   do {                                       \

@@ -234,11 +234,6 @@ __device__ __forceinline__ void read_frags(const float* __restrict__ S, int oute
   }
 }
 
-// Workgroups are dispatched to the 8 XCDs round-robin (workgroup w runs on
-// XCD w % 8), and each XCD has its own L2.  Renumbering so that XCD x
-// receives the contiguous run [x*n/8, (x+1)*n/8) of the grouped tile order
-// keeps the tiles that share A rows and B columns on one L2.  A bijection on
-// [0, n): ids past the last multiple of 8 keep their number.
 // Waves per workgroup: WR rows x 2 columns, each wave keeping a
 // (BM / WR) x (BN / 2) sub-tile: 2 x 2 waves, or 4 x 2 for the 8-wave
 // 256-row tiles (B shared by four waves).
@@ -247,13 +242,6 @@ constexpr int gemm_threads(int wr) { return wr * 128; }
 // accumulators alone take 96 registers or more), smaller ones four.
 constexpr int gemm_waves_per_simd(int bm, int bn, int wr) {
   return (bm / wr) * (bn / 2) >= 64 * 96 ? 2 : 4;
-}
-
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_tile(int bid, int n) {
-  const int full = n - n % kXcds;
-  if (bid >= full) return bid;
-  return (bid % kXcds) * (full / kXcds) + bid / kXcds;
 }
 
 template <int BM, int BN, int WR, bool TA, bool TB, bool EDGE, bool XF = false>

@@ -1,6 +1,6 @@
 // What the GEMM kernels of gemm.hip (float products) and gemm_split.h (split
-// products) share: their arguments, the activation epilogue and the sum of
-// split-K partials.
+// products) share: their arguments, the order of the tiles, the activation
+// epilogue and the sum of split-K partials.
 #pragma once
 
 #include "common.h"
@@ -54,6 +54,18 @@ template <int V>
 struct IConst {
   static constexpr int value = V;
 };
+
+// Workgroups are dispatched to the 8 XCDs round-robin (workgroup w runs on
+// XCD w % 8), and each XCD has its own L2.  Renumbering so that XCD x
+// receives the contiguous run [x*n/8, (x+1)*n/8) of the grouped tile order
+// keeps the tiles that share A rows and B columns on one L2.  A bijection on
+// [0, n): ids past the last multiple of 8 keep their number.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int xcd_tile(int bid, int n) {
+  const int full = n - n % kXcds;
+  if (bid >= full) return bid;
+  return (bid % kXcds) * (full / kXcds) + bid / kXcds;
+}
 
 // The activation epilogue, shared by the GEMM and the split-K sum.
 __device__ __forceinline__ float epilogue_act(const GemmArgs& g, int64_t row, int64_t col,

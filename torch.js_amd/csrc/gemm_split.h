@@ -1,10 +1,11 @@
 // fp32 GEMM on the CDNA4 bf16 matrix cores: products of floats split into
 // three bf16 parts.  Serves the products that no gradient is taken through
-// and large weight gradients (tjh_gemm_split); gemm.hip's float matrix cores
-// serve the other recorded ones, whose roundings a training run depends on:
-// AdamW's g / (|g| + eps) amplifies a change of all of them to 2e-5 in the
-// second step's gradients of GPT-2, in which the float path itself is
-// 1.6e-5 from 64 bits.
+// and the weight gradients of vocabulary tables (tjh_gemm_split); gemm.hip's
+// float matrix cores serve the other recorded ones, whose roundings a
+// training run depends on: AdamW's g / (|g| + eps) amplifies a change of all
+// of them to 2e-5 in the second step's gradients of GPT-2, in which the float
+// path itself is 1.6e-5 from 64 bits.  A result under no_grad therefore
+// differs from the recorded one by roundings.
 //
 // Stands for matmul.wgsl:17-50 behind Tensor.matmul / mm and nn.Linear
 // (Tensor.ts:2132-2331, src/nn/linear.ts:43-66) under no_grad.
@@ -237,18 +238,6 @@ struct Tile {
     }
   }
 };
-
-// Workgroups are dispatched to the 8 XCDs round-robin (workgroup w runs on
-// XCD w % 8), and each XCD has its own L2.  Renumbering so that XCD x
-// receives the contiguous run [x*n/8, (x+1)*n/8) of the grouped tile order
-// keeps the tiles that share A rows and B columns on one L2.  A bijection on
-// [0, n): ids past the last multiple of 8 keep their number.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_tile(int bid, int n) {
-  const int full = n - n % kXcds;
-  if (bid >= full) return bid;
-  return (bid % kXcds) * (full / kXcds) + bid / kXcds;
-}
 
 // Wave tiles that keep 96 accumulator registers or more run two waves per
 // SIMD (256 registers each), smaller ones three or more.
@@ -663,17 +652,3 @@ void launch_split(const GemmArgs& g, dim3 grid, int ta, int tb, bool edge) {
 }
 
 }  // namespace tjh
-
-/* tjh_gemm (batch 1) for a result that no gradient is taken through: float
- * products formed from three bf16 parts of each operand.  Its error against
- * 64 bits is no larger than tjh_gemm's, but its roundings are others.  (Elements under
- * 2^-109 in magnitude keep an absolute error of up to 2^-134.)
- * act 0: nothing; 1: C = GELU(v); 3: C = residual + v, with residual [M][N]
- * at row stride ldr, not overlapping C.  bias_mode 0 to 3 as tjh_gemm, 3
- * (bias receives the row sums of op(A)) with act 0 only.
- * For the Python host, which knows what is recorded; not part of the
- * library's declared interface. */
-extern "C" int tjh_gemm_split(int transA, int transB, int64_t M, int64_t N, int64_t K, float alpha,
-                              const float* A, int64_t lda, const float* B, int64_t ldb, float beta,
-                              float* C, int64_t ldc, const float* bias, int bias_mode,
-                              const float* residual, int64_t ldr, int act);

@@ -767,9 +767,10 @@ def scaled_dot_product_attention(query, key, value, attn_mask=None, dropout_p=0.
     # the backward reads lse; without one the keys may be split over workgroups
     lse = empty((B, H, Tq)) if _T._recorded(query, key, value) else None
     L.check(L.lib().tjh_sdpa_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                     lse.data_ptr() if lse is not None else None, B, H, Tq, Tk, D, L.i64arr(q._strides[:3]),
-                                     L.i64arr(k._strides[:3]), L.i64arr(v._strides[:3]),
-                                     L.i64arr(o._strides[:3]), sc, 1 if is_causal else 0), "sdpa")
+                                     lse.data_ptr() if lse is not None else None, B, H, Tq, Tk, D,
+                                     L.i64arr(q._strides[:3]), L.i64arr(k._strides[:3]),
+                                     L.i64arr(v._strides[:3]), L.i64arr(o._strides[:3]), sc,
+                                     1 if is_causal else 0), "sdpa")
 
     def grad_like(t):
         Bx, Hx, Tx, Dx = t.shape
