@@ -65,7 +65,6 @@
 
 #include "gemm_args.h"
 #include "kahan.h"
-#include "wave.h"
 
 #include <math.h>
 
@@ -208,9 +207,8 @@ struct Tile {
     }
   }
   // Splits the tile and stores its parts in LDS, `part` bytes apart, outer
-  // index o negated where it is odd.  `top` is raised to the largest
-  // magnitude.
-  __device__ __forceinline__ void store(char* __restrict__ S, int part, float& top) const {
+  // index o negated where it is odd.
+  __device__ __forceinline__ void store(char* __restrict__ S, int part) const {
 #pragma unroll
     for (int i = 0; i < I; ++i) {
       if (!has(i)) continue;
@@ -223,8 +221,6 @@ struct Tile {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           unsigned a, b, c;
-          // (fmaxf would first quiet each operand)
-          asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(r[i][w][2 * q]), "v"(r[i][w][2 * q + 1]));
           split2(r[i][w][2 * q], r[i][w][2 * q + 1], sign, a, b, c);
           h[q] = a;
           m[q] = b;
@@ -310,7 +306,6 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   constexpr int PA = BM * BK * 2, PB = BN * BK * 2, BUF = 3 * (PA + PB);
   static_assert(FM >= 1 && FN >= 1 && FM * 32 == WM && FN * 32 == WN, "tile");
   __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
-  __shared__ float tops[WR * WC];  // each wave's largest operand
 
   // Wave priority: the prologue and the epilogue run at raised priority.
   // Where two workgroups share a CU, at equal priority the one in its
@@ -373,12 +368,11 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
     xa.load(A, g.lda, g.M, m0, k0);
     xb.load(B, g.ldb, g.N, n0, k0);
   };
-  float top = 0.f;
   auto stage = [&](int64_t t, TileA& xa, TileB& xb) {
     char* S = lds + (t & 1) * BUF;
     if (TA && row_sums) xa.sum(rsum);
-    xa.store(S, PA, top);
-    xb.store(S + 3 * PA, PB, top);
+    xa.store(S, PA);
+    xb.store(S + 3 * PA, PB);
   };
   // the six products of a K tile, the smallest terms first
   auto compute = [&](int64_t t) {
@@ -464,9 +458,6 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   }
 
   __builtin_amdgcn_s_setprio(3);
-  top = wave_max(top);
-  if (lane == 0) tops[wid] = top;
-  __syncthreads();
   if (TA && row_sums) {
     // the two k halves of a row are in two lanes, added with what their
     // compensations hold (50257 rows over 8192: 3.9e-8 off 64 bits, 5.6e-8 by
@@ -541,30 +532,24 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   // 3072 x 768 takes 75 us, with a NaN in every row 243 us (11.3 ms by
   // multiply-adds one after the other, 89 us on gemm.hip's tiles).
   // Operands under 2^-109, too: what the parts lose of them is 2^-134 a term
-  // times the other operand, which only sums under `least` can show; a block
-  // that has such a sum looks for such operands.  (Following the largest
-  // operand for it costs 1.5% of a large product.)
-  float least = 0.f;
-#pragma unroll
-  for (int w = 0; w < WR * WC; ++w) least = fmaxf(least, tops[w]);
-  least *= (float)(kend - kbeg) * 0x1p-108f;
+  // times the other operand.  A block with a sum under 2^-60 looks for such
+  // operands; a larger sum shows nothing of them unless the other operand
+  // times the number of terms exceeds 2^48.  (Following the largest operand
+  // through the K steps, to know, took 1 to 4%.)
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      float z0 = 0.f, z1 = 0.f;
+      float z0 = 0.f, z1 = 0.f, low_sum = INFINITY;
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         z0 = __builtin_fmaf(acc[i][j][r], 0.f, z0);
         z1 = __builtin_fmaf(acc[i][j][r + 1], 0.f, z1);
+        asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(low_sum) : "v"(acc[i][j][r]), "v"(acc[i][j][r + 1]));
       }
       bool again = !(z0 + z1 == 0.f);
       const int64_t row = m0 + wm * WM + i * 32 + l32, col = n0 + wn * WN + j * 32 + l32;
-      float least_sum = INFINITY;
-#pragma unroll
-      for (int r = 0; r < 16; r += 2)
-        asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(least_sum) : "v"(acc[i][j][r]), "v"(acc[i][j][r + 1]));
-      if (__any(least_sum < least))
+      if (__any(low_sum < 0x1p-60f))
         again |= tiny_operand<TA>(g.A, g.lda, row, g.M, h, kbeg, kend) ||
                  tiny_operand<!TB>(g.B, g.ldb, col, g.N, h, kbeg, kend);
       if (__any(again)) {
