@@ -66,8 +66,6 @@
 #include "gemm_args.h"
 #include "kahan.h"
 
-#include <math.h>
-
 namespace tjh {
 
 // ------------------------------------------------------- the operand split
@@ -76,7 +74,7 @@ namespace tjh {
 // bfloat16 of what is left.  Three times eight significant bits hold the 24
 // of a float: the sum is exact while the parts stay above the smallest
 // bfloat16 (2^-133; the matrix cores keep subnormal operands), so for |x| >=
-// 2^-109; below, an absolute error of at most 2^-134 remains (tiny_operand).
+// 2^-109; below, an absolute error of at most 2^-134 remains (kTinySum).
 // For 1 <= |x| < 2, |m| <= 2^-8 and |l| <= 2^-17, so
 // of the nine products of two split numbers the three not formed (m l, l m,
 // l l) are at most 2^-24 + 2^-34 of the product, one float rounding of it
@@ -241,22 +239,10 @@ constexpr int gemm_waves_per_simd(int wm, int wn) {
   return wm * wn >= 64 * 64 ? 2 : wm * wn >= 64 * 32 ? 3 : 4;
 }
 
-// Whether outer index o (clamped to n) of an operand, stored [k][outer] (KT)
-// or [outer][k], has a value but zero under 2^-109 among its k = kbeg + h,
-// + 2, ...
-template <bool KT>
-__device__ __forceinline__ bool tiny_operand(const float* __restrict__ P, int64_t ld, int64_t o,
-                                             int64_t n, int h, int64_t kbeg, int64_t kend) {
-  if (o >= n) o = n - 1;
-  const float* __restrict__ p = KT ? P + o : P + o * ld;
-  bool tiny = false;
-#pragma unroll 4
-  for (int64_t k = kbeg + h; k < kend; k += 2) {
-    const float x = __builtin_fabsf(p[KT ? k * ld : k]);
-    tiny |= x > 0.f && x < 0x1p-109f;
-  }
-  return tiny;
-}
+// A sum other than zero of less than this magnitude (as the bits of a float
+// shifted left, less one, so that zero is the largest), 2^-75, can show what
+// operands under 2^-109 lost.
+constexpr unsigned kTinySum = ((127u - 75) << 24) - 1;
 
 // The 32 x 32 block of products over [kbeg, kend) that holds row `row` (of
 // this lane's A value) and column `col` (of its B value; both clamped to the
@@ -531,27 +517,27 @@ __global__ __launch_bounds__(WR * WC * 64, gemm_waves_per_simd(BM / WR, BN / WC)
   // float arithmetic.  0 * x is 0 for finite x and NaN otherwise.  2048 x
   // 3072 x 768 takes 75 us, with a NaN in every row 243 us (11.3 ms by
   // multiply-adds one after the other, 89 us on gemm.hip's tiles).
-  // Operands under 2^-109, too: what the parts lose of them is 2^-134 a term
-  // times the other operand.  A block with a sum under 2^-60 looks for such
-  // operands; a larger sum shows nothing of them unless the other operand
-  // times the number of terms exceeds 2^48.  (Following the largest operand
-  // through the K steps, to know, took 1 to 4%.)
+  // So are blocks with a sum under 2^-75 but not zero: what the parts lose of
+  // operands under 2^-109 is 2^-134 a term times the other operand, which
+  // larger sums show nothing of unless that operand times the number of terms
+  // exceeds 2^33.  (2048 x 3072 x 768 with operands of 1e-12 takes 225 us.
+  // Following the largest operand through the K steps, to know, took 1 to 4%;
+  // looking for tiny operands took longer than the block.)
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      float z0 = 0.f, z1 = 0.f, low_sum = INFINITY;
+      float z0 = 0.f, z1 = 0.f;
+      unsigned low_sum = ~0u;
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         z0 = __builtin_fmaf(acc[i][j][r], 0.f, z0);
         z1 = __builtin_fmaf(acc[i][j][r + 1], 0.f, z1);
-        asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(low_sum) : "v"(acc[i][j][r]), "v"(acc[i][j][r + 1]));
+        low_sum = min(low_sum, min((__float_as_uint(acc[i][j][r]) << 1) - 1,
+                                   (__float_as_uint(acc[i][j][r + 1]) << 1) - 1));
       }
-      bool again = !(z0 + z1 == 0.f);
+      const bool again = !(z0 + z1 == 0.f) || low_sum < kTinySum;
       const int64_t row = m0 + wm * WM + i * 32 + l32, col = n0 + wn * WN + j * 32 + l32;
-      if (__any(low_sum < 0x1p-60f))
-        again |= tiny_operand<TA>(g.A, g.lda, row, g.M, h, kbeg, kend) ||
-                 tiny_operand<!TB>(g.B, g.ldb, col, g.N, h, kbeg, kend);
       if (__any(again)) {
         acc[i][j] = float_block<TA, TB>(g, row, col, h, kbeg, kend);
 #pragma unroll
